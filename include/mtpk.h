@@ -450,6 +450,22 @@ int mtpk_delta_rule(float* state, int64_t slots_total, const int64_t* slot, int6
                     const float* k, const float* v, const float* g, const float* beta,
                     const int64_t* lengths, float* out, void* stream);
 
+/* The same with a workspace for calls of many steps (a prompt's rows): where
+ * mtpk_delta_rule_workspace_bytes is positive (k_dim 128, v_dim a multiple of 64, and steps enough for the rows),
+ * 64 steps at a time become fp32 matrix products and only every 64th step waits for the state;
+ * a (row, head) whose k is longer than 1, whose g is positive, whose beta lies outside [0, 1] or
+ * whose v, k, g or beta is not finite runs step by step as before. The bytes cover one row or
+ * more; rows run in groups that fit, so a larger workspace takes fewer launches. workspace is
+ * 256-byte aligned. Where it is 0, or with operands that are not 16-byte aligned, the call is
+ * mtpk_delta_rule (workspace unused, may be NULL). */
+int64_t mtpk_delta_rule_workspace_bytes(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads,
+                                        int64_t k_dim, int64_t v_dim, int want_out);
+int mtpk_delta_rule_ws(float* state, int64_t slots_total, const int64_t* slot, int64_t rows, int64_t t,
+                       int64_t heads, int64_t qk_heads, int64_t k_dim, int64_t v_dim, const float* q,
+                       const float* k, const float* v, const float* g, const float* beta,
+                       const int64_t* lengths, float* out, void* workspace, int64_t workspace_bytes,
+                       void* stream);
+
 /* Verify-row preparation of a Gated DeltaNet layer, replacing the torch chain of
  * `deltanet_verify` (model.py:3738-3905) between the in-projection and the recurrence: proj
  * [batch * t, proj_stride] (model dtype f32|bf16; per row qkv [C], z [v_heads * v_dim],
@@ -491,6 +507,15 @@ int mtpk_deltanet_commit(float* state, int64_t slots_total, const int64_t* slot,
                          int conv_dtype, int64_t conv_slots_total, const void* proj,
                          int64_t proj_stride, const int64_t* conv_idx, int64_t channels, int64_t k1,
                          void* stream);
+/* The same with mtpk_delta_rule_ws's workspace (want_out = 0); without one it is
+ * mtpk_deltanet_commit. */
+int mtpk_deltanet_commit_ws(float* state, int64_t slots_total, const int64_t* slot, int64_t rows,
+                            int64_t t, int64_t heads, int64_t qk_heads, int64_t k_dim, int64_t v_dim,
+                            const float* q, const float* k, const float* v, const float* g,
+                            const float* beta, const int64_t* lengths, void* conv_state,
+                            int conv_dtype, int64_t conv_slots_total, const void* proj,
+                            int64_t proj_stride, const int64_t* conv_idx, int64_t channels, int64_t k1,
+                            void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ---------------------------------------------------------------- skinny bf16 GEMM
  * y[M, N] = x[M, K] . w[N, K]^T for M <= 256 token rows, bf16 in, fp32 accumulation: the

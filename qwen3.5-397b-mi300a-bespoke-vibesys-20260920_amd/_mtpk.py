@@ -134,6 +134,12 @@ _SIGNATURES: dict[str, tuple[object, list]] = {
          c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_void_p,
          c_int64, c_void_p, c_int64, c_int64, c_void_p],
     ),
+    "mtpk_deltanet_commit_ws": (
+        c_int,
+        [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p,
+         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_void_p,
+         c_int64, c_void_p, c_int64, c_int64, c_void_p, c_int64, c_void_p],
+    ),
     "mtpk_moe_dense_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int64]),
     "mtpk_moe_dense": (
         c_int,
@@ -214,6 +220,12 @@ _SIGNATURES: dict[str, tuple[object, list]] = {
         c_int,
         [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p,
          c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p],
+    ),
+    "mtpk_delta_rule_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_int]),
+    "mtpk_delta_rule_ws": (
+        c_int,
+        [c_void_p, c_int64, c_void_p, c_int64, c_int64, c_int64, c_int64, c_int64, c_int64, c_void_p,
+         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_void_p],
     ),
     "mtpk_attention_splits": (c_int, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int64]),
     "mtpk_attention_workspace_bytes": (c_int64, [c_int64, c_int64, c_int64, c_int64, c_int64, c_int]),

@@ -17,6 +17,7 @@
 // state is not written. Commit mode: row j replays its accepted prefix, min(lengths[j], t)
 // steps, and stores the advanced state over its slot (outputs optional).
 
+#include "mtpk_deltanet_chunk.h"
 #include "mtpk_device.h"
 #include "mtpk_host.h"
 
@@ -157,7 +158,7 @@ __device__ inline float group_sum(float x) {
 }
 
 template <int KG, bool OUT, bool COMMIT>
-__device__ inline void delta_rule_kg_body(
+__device__ __forceinline__ void delta_rule_kg_body(
     int bid, float* __restrict__ state, int64_t slots_total, const int64_t* __restrict__ slot, int t,
     int heads, int rep, int dv, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ g, const float* __restrict__ beta,
@@ -319,6 +320,93 @@ int launch_delta_rule_mode(float* state, int64_t slots_total, const int64_t* slo
                                              lengths, out, st);
   return launch_delta_rule<DK, false, true>(state, slots_total, slot, rows, t, heads, rep, dv, q, k, v, g, beta,
                                             lengths, nullptr, st);
+}
+
+// The (row, head) matrices that the chunk scan left, step by step.
+template <bool OUT, bool COMMIT>
+__global__ __launch_bounds__(kWave, (OUT && COMMIT) ? 2 : 3) void k_delta_rule_rest(
+    float* __restrict__ state, int64_t slots_total, const int64_t* __restrict__ slot, int t,
+    int heads, int rep, int dv, const float* __restrict__ q, const float* __restrict__ k,
+    const float* __restrict__ v, const float* __restrict__ g, const float* __restrict__ beta,
+    const int64_t* __restrict__ lengths, float* __restrict__ out, const int32_t* __restrict__ odd,
+    int nch) {
+  const int bh = (int)blockIdx.x / (dv / (4 * kWave / kDnKG));
+  if (!dn_left_over(odd, nch, bh, lengths, bh / heads, t)) return;  // uniform
+  delta_rule_kg_body<kDnKG, OUT, COMMIT>((int)blockIdx.x, state, slots_total, slot, t, heads, rep, dv,
+                                         q, k, v, g, beta, lengths, out);
+}
+
+constexpr int64_t kDnChunkWsBytes = int64_t(256) << 20;
+
+// Workspace of one row of a chunked call (a multiple of 256 bytes).
+int64_t dn_chunk_row_bytes(int64_t t, int64_t heads, int64_t qk_heads, bool want_out) {
+  const int64_t nch = (t + kDnChunk - 1) / kDnChunk, m = want_out ? 2 : 1;
+  return qk_heads * nch * (m + 1) * kDnRowTiles * kDnTile * 4 +
+         heads * nch * (m * kDnSqTiles * kDnTile + 2 * kDnChunk) * 4 + align256(heads * nch * 4);
+}
+
+// Whether a call's sizes are for the chunk form: its shapes (32-bit byte offsets inside a row), and
+// the faster of the two by these fits, in us. m counts matrices of 64 heads of 128 x 128. Step by
+// step a step takes 2.1 us (1.5 read back to back) while every wave is resident and more as rows are
+// added; the chunks cost two launches and 64 steps' products, which fill the chip from m = 1 on.
+// Step by step / chunks, with outputs: m = 1, 24 steps 55 / 30, 1500 steps 2286 / 180; m = 4, 24
+// steps 67 / 67, 128 steps 319 / 120; m = 16, 48 steps 163 / 204, 128 steps 430 / 369; m = 48, 128
+// steps 1011 / 1121. Commits: m = 1, 24 steps 26 / 25, 1500 steps 1637 / 116; m = 4, 48 steps
+// 60 / 52; m = 16, 128 steps 183 / 238.
+bool dn_chunk_fits(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads, int64_t k_dim, int64_t v_dim,
+                   bool want_out) {
+  if (k_dim != kDnChunkDk || v_dim % (4 * kWave / kDnKG) != 0 ||
+      (t + kDnChunk) * (qk_heads * k_dim > heads * v_dim ? qk_heads * k_dim : heads * v_dim) * 4 >=
+          (int64_t(1) << 31))
+    return false;
+  const double m = (double)rows * heads * v_dim / (64 * 128), n = (double)((t + kDnChunk - 1) / kDnChunk);
+  const double least = want_out ? 6.0 : 3.6, full = m * (want_out ? 10.3 : 6.2);
+  const double chunks = 20.0 + n * (full > least ? full : least);
+  const double steps = t * (want_out ? 2.1 + 0.075 * m : 0.95 + 0.03 * m);
+  return chunks < steps;
+}
+
+DnChunkWs dn_chunk_ws(void* workspace, int64_t rows, int64_t t, int64_t heads, int64_t qk_heads,
+                      bool want_out) {
+  const int64_t nch = (t + kDnChunk - 1) / kDnChunk;
+  const int64_t kq = rows * qk_heads * nch * kDnRowTiles * kDnTile, slabs = rows * heads * nch;
+  const int64_t sq = slabs * kDnSqTiles * kDnTile;
+  DnChunkWs w{};
+  float* p = static_cast<float*>(workspace);
+  auto take = [&](int64_t n) {
+    float* const at = p;
+    p += n;
+    return at;
+  };
+  w.kr = take(kq);
+  w.kc = take(kq);
+  w.tm = take(sq);
+  if (want_out) {
+    w.qr = take(kq);
+    w.am = take(sq);
+  }
+  w.eg = take(slabs * kDnChunk);
+  w.dg = take(slabs * kDnChunk);
+  w.odd = reinterpret_cast<int32_t*>(p);
+  return w;
+}
+
+// The chunk launches of `rows` rows: prep and scan. The caller launches what the scan left.
+template <bool OUT, bool COMMIT>
+int launch_dn_chunks(float* state, int64_t slots_total, const int64_t* slot, int rows, int t, int heads,
+                     int qk_heads, int dv, const float* q, const float* k, const float* v,
+                     const float* g, const float* beta, const int64_t* lengths, float* out,
+                     const DnChunkWs& ws, hipStream_t st) {
+  const int nch = (t + kDnChunk - 1) / kDnChunk;
+  const int64_t pg = (int64_t)rows * qk_heads * nch, sg = (int64_t)rows * heads * (dv / kDnScanCols);
+  if (pg > INT32_MAX || sg > INT32_MAX) return MTPK_EINVAL;
+  hipLaunchKernelGGL((k_dn_chunk_prep<OUT>), dim3((unsigned)pg), dim3(256), 0, st, t, heads, qk_heads, dv, nch, q,
+                     k, v, g, beta, lengths, ws);
+  const int rc = status_of(hipGetLastError());
+  if (rc) return rc;
+  hipLaunchKernelGGL((k_dn_chunk_scan<OUT, COMMIT>), dim3((unsigned)sg), dim3(256 * kDnScanTiles), 0, st, state, slots_total,
+                     slot, t, heads, qk_heads, dv, nch, v, lengths, out, ws, rows * heads);
+  return status_of(hipGetLastError());
 }
 
 // ---------------------------------------------------------------- verify-row preparation
@@ -587,6 +675,90 @@ int mtpk_deltanet_commit(float* state, int64_t slots_total, const int64_t* slot,
                      (hipStream_t)stream, state, slots_total, slot, (int)t, (int)heads,
                      (int)(heads / qk_heads), (int)v_dim, q, k, v, g, beta, lengths, dr, cj);
   return status_of(hipGetLastError());
+}
+
+int64_t mtpk_delta_rule_workspace_bytes(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads,
+                                        int64_t k_dim, int64_t v_dim, int want_out) {
+  if (rows <= 0 || t < 1 || t > INT32_MAX / 2 || heads <= 0 || qk_heads <= 0 || heads % qk_heads ||
+      v_dim <= 0 || v_dim > 4096)
+    return 0;
+  if (!dn_chunk_fits(rows, t, heads, qk_heads, k_dim, v_dim, want_out != 0)) return 0;
+  const int64_t one = dn_chunk_row_bytes(t, heads, qk_heads, want_out != 0);
+  const int64_t fit = kDnChunkWsBytes / one;
+  return one * (fit < 1 ? 1 : fit < rows ? fit : rows);
+}
+
+int mtpk_delta_rule_ws(float* state, int64_t slots_total, const int64_t* slot, int64_t rows, int64_t t,
+                       int64_t heads, int64_t qk_heads, int64_t k_dim, int64_t v_dim, const float* q,
+                       const float* k, const float* v, const float* g, const float* beta,
+                       const int64_t* lengths, float* out, void* workspace, int64_t workspace_bytes,
+                       void* stream) {
+  if (!state || !q || !k || !v || !g || !beta || slots_total <= 0 || (!slot && slots_total < rows) ||
+      (!lengths && !out) || slots_total * heads * k_dim * v_dim >= (int64_t(1) << 40) || !workspace ||
+      (reinterpret_cast<uintptr_t>(workspace) & 255u) || !aligned16(state) || !aligned16(q) ||
+      !aligned16(k) || !aligned16(v) ||
+      mtpk_delta_rule_workspace_bytes(rows, t, heads, qk_heads, k_dim, v_dim, out != nullptr) <= 0)
+    return mtpk_delta_rule(state, slots_total, slot, rows, t, heads, qk_heads, k_dim, v_dim, q, k, v, g,
+                           beta, lengths, out, stream);
+  const int64_t one = dn_chunk_row_bytes(t, heads, qk_heads, out != nullptr), fit = workspace_bytes / one;
+  if (fit < 1) return MTPK_EINVAL;
+  const hipStream_t st = (hipStream_t)stream;
+  const int rep = (int)(heads / qk_heads), nch = (int)((t + kDnChunk - 1) / kDnChunk);
+  for (int64_t r0 = 0; r0 < rows; r0 += fit) {  // as many rows at once as the workspace holds
+    const int r = (int)(rows - r0 < fit ? rows - r0 : fit);
+    const DnChunkWs ws = dn_chunk_ws(workspace, r, t, heads, qk_heads, out != nullptr);
+    const int64_t qo = r0 * t * qk_heads * k_dim, vo = r0 * t * heads * v_dim, go = r0 * t * heads;
+    const int64_t* const ln = lengths ? lengths + r0 : nullptr;
+    float* const o = out ? out + vo : nullptr;
+    float* const stt = slot ? state : state + r0 * heads * k_dim * v_dim;  // no slots: row j is slot j
+    const int64_t* const sl = slot ? slot + r0 : nullptr;
+    const int64_t total = slot ? slots_total : slots_total - r0;
+    int rc;
+    const unsigned grid = (unsigned)(r * heads * (v_dim / (4 * kWave / kDnKG)));
+#define MTPK_DNC(OUT_, COMMIT_)                                                                      \
+  rc = launch_dn_chunks<OUT_, COMMIT_>(stt, total, sl, r, (int)t, (int)heads,                       \
+                                       (int)qk_heads, (int)v_dim, q + qo, k + qo, v + vo, g + go,    \
+                                       beta + go, ln, o, ws, st);                                    \
+  if (rc) return rc;                                                                                 \
+  hipLaunchKernelGGL((k_delta_rule_rest<OUT_, COMMIT_>), dim3(grid), dim3(kWave), 0, st, stt,        \
+                     total, sl, (int)t, (int)heads, rep, (int)v_dim, q + qo, k + qo,    \
+                     v + vo, g + go, beta + go, ln, o, ws.odd, nch);
+    if (!lengths) {
+      MTPK_DNC(true, false)
+    } else if (out) {
+      MTPK_DNC(true, true)
+    } else {
+      MTPK_DNC(false, true)
+    }
+#undef MTPK_DNC
+    rc = status_of(hipGetLastError());
+    if (rc) return rc;
+  }
+  return 0;
+}
+
+int mtpk_deltanet_commit_ws(float* state, int64_t slots_total, const int64_t* slot, int64_t rows,
+                            int64_t t, int64_t heads, int64_t qk_heads, int64_t k_dim, int64_t v_dim,
+                            const float* q, const float* k, const float* v, const float* g,
+                            const float* beta, const int64_t* lengths, void* conv_state,
+                            int conv_dtype, int64_t conv_slots_total, const void* proj,
+                            int64_t proj_stride, const int64_t* conv_idx, int64_t channels, int64_t k1,
+                            void* workspace, int64_t workspace_bytes, void* stream) {
+  if (!lengths || !slot ||
+      mtpk_delta_rule_workspace_bytes(rows, t, heads, qk_heads, k_dim, v_dim, 0) <= 0)
+    return mtpk_deltanet_commit(state, slots_total, slot, rows, t, heads, qk_heads, k_dim, v_dim, q, k, v,
+                                g, beta, lengths, conv_state, conv_dtype, conv_slots_total, proj,
+                                proj_stride, conv_idx, channels, k1, stream);
+  // the conv window's argument checks come before the state's launches, as in the one-launch commit
+  if (!conv_state || !proj || !conv_idx || (conv_dtype != MTPK_F32 && conv_dtype != MTPK_BF16) ||
+      channels < 1 || k1 < 1 || k1 > kConvMaxK1 || proj_stride < channels || conv_slots_total < 1 ||
+      rows * channels > INT32_MAX)
+    return MTPK_EINVAL;
+  const int rc = mtpk_delta_rule_ws(state, slots_total, slot, rows, t, heads, qk_heads, k_dim, v_dim, q, k,
+                                    v, g, beta, lengths, nullptr, workspace, workspace_bytes, stream);
+  if (rc) return rc;
+  return mtpk_conv_commit(conv_state, conv_dtype, slot, conv_slots_total, proj, proj_stride, conv_idx, rows,
+                          channels, k1, t, stream);
 }
 
 }  // extern "C"

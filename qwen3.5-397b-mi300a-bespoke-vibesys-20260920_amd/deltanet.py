@@ -19,6 +19,13 @@ import torch
 import _mtpk
 
 
+def _steps_workspace(rows: int, t: int, heads: int, qk_heads: int, k_dim: int, v_dim: int, want_out: bool,
+                     device: torch.device) -> torch.Tensor | None:
+    """Scratch of a call of many steps (`mtpk_delta_rule_workspace_bytes`), None where it takes none."""
+    n = int(_mtpk.lib().mtpk_delta_rule_workspace_bytes(rows, t, heads, qk_heads, k_dim, v_dim, int(want_out)))
+    return torch.empty(n, dtype=torch.uint8, device=device) if n > 0 else None
+
+
 def delta_rule(state: torch.Tensor, slots: torch.Tensor | None, q: torch.Tensor, k: torch.Tensor,
                v: torch.Tensor, g: torch.Tensor, beta: torch.Tensor,
                lengths: torch.Tensor | None = None, *, want_out: bool = True) -> torch.Tensor | None:
@@ -59,11 +66,13 @@ def delta_rule(state: torch.Tensor, slots: torch.Tensor | None, q: torch.Tensor,
         raise ValueError("verify mode (no lengths) produces only outputs")
     f32 = [x.to(torch.float32).contiguous() for x in (q, k, v, g, beta)]
     out = torch.empty(rows, t, heads, v_dim, dtype=torch.float32, device=device) if want_out else None
+    ws = _steps_workspace(rows, t, heads, qk_heads, k_dim, v_dim, want_out, device)
     _mtpk.check(
-        _mtpk.lib().mtpk_delta_rule(
+        _mtpk.lib().mtpk_delta_rule_ws(
             state.data_ptr(), n_slots, _mtpk.ptr(slots), rows, t, heads, qk_heads, k_dim, v_dim,
-            *(x.data_ptr() for x in f32), _mtpk.ptr(lengths), _mtpk.ptr(out), _mtpk.stream_of(device)),
-        "mtpk_delta_rule",
+            *(x.data_ptr() for x in f32), _mtpk.ptr(lengths), _mtpk.ptr(out), _mtpk.ptr(ws),
+            0 if ws is None else ws.numel(), _mtpk.stream_of(device)),
+        "mtpk_delta_rule_ws",
     )
     return out
 
@@ -98,11 +107,13 @@ def commit(state: torch.Tensor, conv_state: torch.Tensor, slots: torch.Tensor, q
     sl = slots.to(device, torch.int64).contiguous()
     ln = lengths.to(device, torch.int64).contiguous()
     f32 = [x.to(torch.float32).contiguous() for x in (q, k, v, g, beta)]
-    _mtpk.check(_mtpk.lib().mtpk_deltanet_commit(
+    ws = _steps_workspace(rows, t, heads, qk_heads, k_dim, v_dim, False, device)
+    _mtpk.check(_mtpk.lib().mtpk_deltanet_commit_ws(
         state.data_ptr(), n_slots, sl.data_ptr(), rows, t, heads, qk_heads, k_dim, v_dim,
         *(x.data_ptr() for x in f32), ln.data_ptr(), conv_state.data_ptr(),
         _mtpk.float_code(conv_state.dtype), conv_state.shape[0], proj.data_ptr(), rs, ix.data_ptr(),
-        channels, k1, _mtpk.stream_of(device)), "mtpk_deltanet_commit")  # fmt: skip
+        channels, k1, _mtpk.ptr(ws), 0 if ws is None else ws.numel(), _mtpk.stream_of(device)),
+        "mtpk_deltanet_commit_ws")  # fmt: skip
 
 
 def prep(proj: torch.Tensor, conv_state: torch.Tensor, slots: torch.Tensor, conv_w: torch.Tensor,

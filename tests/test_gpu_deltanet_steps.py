@@ -1,0 +1,120 @@
+"""Calls of many delta-rule steps (`mtpk_delta_rule_ws`: 64 steps at a time as fp32 matrix products)
+against the float64 oracle, at the edges of the 64-step chunks, with the rows and heads that
+run step by step instead.
+
+Bar: every output is a sum of at most 128 fp32 products of a state that 64-step sums build up; the
+decays are at most 1 and k at most unit length, so errors do not grow with the steps: 1e-5 of the
+largest value, about 100 fp32 roundings."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import deltanet
+from oracle import deltanet_ref as dn
+
+from .test_gpu_deltanet import _case, _dev
+
+pytestmark = pytest.mark.gpu
+
+
+def _close(got, want):
+    assert np.abs(got - want).max() <= 1e-5 * np.abs(want).max(), np.abs(got - want).max() / np.abs(want).max()
+
+
+@pytest.mark.parametrize("t,heads,qk_heads,dv,rows", [
+    (12, 2, 1, 128, 2),  # too few steps for the chunk form
+    (24, 2, 1, 128, 2), (63, 4, 4, 64, 1), (64, 3, 1, 128, 2), (65, 8, 2, 128, 1), (128, 5, 1, 192, 2),
+    (200, 4, 2, 128, 3),
+])
+def test_many_steps_match_the_oracle(dev, t, heads, qk_heads, dv, rows) -> None:
+    pool, slots, q, k, v, g, beta = _case(t + heads, rows + 2, heads, qk_heads, 128, dv, rows, t)
+    g[:, ::7] *= 60  # decays that forget the state, next to ones that keep it
+    args = _dev(dev, pool, slots.astype(np.int64), q, k, v, g, beta)
+    _, want = dn.delta_rule_rows(pool, slots, q, k, v, g, beta)
+    _close(deltanet.delta_rule(*args).cpu().numpy(), want)
+    assert torch.equal(args[0].cpu(), torch.from_numpy(pool))  # verify leaves the state
+    lengths = np.array([t, t - 1, 0, -3][:rows] if rows > 1 else [t - 2], np.int64)
+    want_pool, _ = dn.delta_rule_rows(pool, slots, q, k, v, g, beta, lengths)
+    out = deltanet.delta_rule(*args, torch.from_numpy(lengths).to(dev)).cpu().numpy()
+    _close(args[0].cpu().numpy(), want_pool)
+    for j in range(rows):
+        n = max(int(lengths[j]), 0)
+        if n:
+            _close(out[j, :n], want[j, :n])
+        else:  # a row that commits nothing, and the slots that no row names, keep their bits
+            assert torch.equal(args[0][slots[j]].cpu(), torch.from_numpy(pool[slots[j]]))
+
+
+def test_rows_without_slots_and_bad_slots(dev) -> None:
+    pool, _, q, k, v, g, beta = _case(5, 4, 4, 2, 128, 128, 3, 70)
+    _, want = dn.delta_rule_rows(pool, np.arange(3), q, k, v, g, beta)
+    args = _dev(dev, pool, q, k, v, g, beta)
+    _close(deltanet.delta_rule(args[0], None, *args[1:]).cpu().numpy(), want)
+    bad = torch.tensor([0, 9, -1], device=dev)
+    out = deltanet.delta_rule(args[0], bad, *args[1:]).cpu().numpy()
+    _close(out[0], want[0])
+    assert not out[1:].any()
+
+
+@pytest.mark.parametrize("what", ["beta", "long_k", "growing", "inf_v", "nan_v", "nan_k", "minus_inf_g"])
+def test_heads_outside_the_chunk_form_run_step_by_step(dev, what) -> None:
+    """One head of one row breaks the chunk form's terms at step 70 of 100: it gets what the
+    step-by-step form gives (bit for bit; NaN only from that step on), the others are unchanged."""
+    pool, slots, q, k, v, g, beta = _case(6, 4, 4, 4, 128, 128, 2, 100)
+    args = _dev(dev, pool, slots.astype(np.int64), q, k, v, g, beta)
+    plain = deltanet.delta_rule(*args)
+    if what == "beta":
+        beta[1, 70, 2] = 1.5
+    elif what == "long_k":
+        k[1, 70, 2] *= 1.2
+    elif what == "growing":
+        g[1, 70, 2] = 0.25
+    elif what == "minus_inf_g":
+        g[1, 70, 2] = -np.inf  # a decay of exactly zero is the chunk form's too
+    else:
+        (v if what.endswith("v") else k)[1, 70, 2, 5] = np.inf if what == "inf_v" else np.nan
+    args = _dev(dev, pool, slots.astype(np.int64), q, k, v, g, beta)
+    got = deltanet.delta_rule(*args)
+    assert torch.equal(got[0], plain[0]) and torch.equal(got[1, :, [0, 1, 3]], plain[1, :, [0, 1, 3]])
+    # the same row in pieces that are too short for the chunk form
+    p, piece = args[0].clone(), []
+    for s in range(0, 100, 10):
+        cut = [x[:, s : s + 10].contiguous() for x in args[2:]]
+        piece.append(deltanet.delta_rule(p, args[1], *cut, torch.full((2,), 10, device=dev)))
+    want = torch.cat(piece, dim=1)[1, :, 2]
+    if what == "minus_inf_g":
+        _close(got[1, :, 2].cpu().numpy(), want.cpu().numpy())
+        return
+    assert torch.equal(torch.isnan(got[1, :, 2]), torch.isnan(want))
+    assert torch.equal(got[1, :, 2].nan_to_num(), want.nan_to_num())
+    assert torch.isfinite(got[1, :70, 2]).all()
+
+
+def test_long_commit_is_the_rule_and_the_window(dev) -> None:
+    """`deltanet.commit` of many steps leaves both pools as the two calls do, also replayed from a graph."""
+    pool, slots, q, k, v, g, beta = _case(8, 4, 4, 2, 128, 128, 2, 90)
+    args = _dev(dev, pool, slots.astype(np.int64), q, k, v, g, beta)
+    ch = 2 * 2 * 128 + 4 * 128
+    conv = torch.randn(4, ch, 3, device=dev).bfloat16()
+    proj = torch.randn(2, 90, ch + 7, device=dev).bfloat16()
+    n = torch.tensor([90, 41], device=dev)
+    idx = (n[:, None] + torch.arange(3, device=dev)).clamp(max=92)
+    p1, c1 = args[0].clone(), conv.clone()
+    deltanet.delta_rule(p1, *args[1:], n, want_out=False)
+    deltanet.conv_commit(c1, args[1], proj, idx, ch)
+    p2, c2 = args[0].clone(), conv.clone()
+    deltanet.commit(p2, c2, *args[1:], n, proj, idx, ch)
+    assert torch.equal(p1, p2) and torch.equal(c1, c2)
+    p3, c3 = args[0].clone(), conv.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        deltanet.commit(p3, c3, *args[1:], n, proj, idx, ch)
+    for _ in range(3):
+        p3.copy_(args[0])
+        c3.copy_(conv)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(p1, p3) and torch.equal(c1, c3)
