@@ -414,17 +414,21 @@ int launch_dn_chunks(float* state, int64_t slots_total, const int64_t* slot, int
 // launch (`deltanet_verify`, model.py:3738-3905, up to `delta_rule_verify_exact`): the depthwise
 // causal conv over the stored window and the new raw columns, SiLU, rounding to the model dtype
 // (the conv output is a model-dtype tensor), the q / k / v split, the q and k L2 norms (q also
-// scaled by k_dim^-1/2), beta = sigmoid(b) and g = -exp(A_log) softplus(a + dt_bias). One wave
-// per (verify row (b, s), head unit), the units being the q heads, then the k heads, then the v
-// heads; lane l holds channels l, l + 64, ... A workgroup is 4 units of one row (grid: rows x
-// units / 4), so the launch has thousands of workgroups and every wave issues all of its loads
-// at once; the workgroups of unit group 0 also write the row's g and beta.
+// scaled by k_dim^-1/2), beta = sigmoid(b) and g = -exp(A_log) softplus(a + dt_bias). A wave takes
+// one head unit (the q heads, then the k heads, then the v heads) over R consecutive rows of a lane:
+// lane l holds channels 2l, 2l + 1 (+ 128), so a raw column is one dword a lane and each column is
+// loaded once for the R rows that see it, all R + conv_k - 1 at once, instead of once per row and
+// tap. The last workgroups write g and beta, a thread per (row, head).
+//
+// 30.8 us at 1500 rows of 12288 channels (111 MB: 3.6 TB/s; the exponentials and divisions of 18 M
+// SiLUs come next) and 8.2 us at 192; a wave per (row, unit) with 16-bit loads took 118 and 21 us.
 //
 // Conv taps run in order j = 0 .. conv_k - 1 as separate products and sums (no fused
 // multiply-add), as the torch form does them.
 constexpr int kPrepThreadsDn = 256;
 constexpr int kConvMaxK1 = 8;  // conv_k - 1 at most
-constexpr int kPrepMaxPerLane = 4;  // head dims up to 256
+constexpr int kPrepMaxDim = 256;  // widest head
+constexpr int kPrepRows = 8;  // rows a wave takes (4 for calls of at most 4 steps)
 
 struct DnPrepArgs {
   const void* proj;       // [B * t, proj_stride] model dtype: qkv (C), z, b (vh), a (vh)
@@ -435,72 +439,173 @@ struct DnPrepArgs {
   const void* conv_w;     // [C, conv_k] model dtype
   const float* a_log;     // [vh] f32
   const float* dt_bias;   // [vh] f32
-  int dt, t, kh, kd, vh, vd, conv_k;
+  int B, dt, t, kh, kd, vh, vd, conv_k;
   float eps, q_scale;
   float *q, *k, *v, *g, *beta;
+  int unit_blocks;        // workgroups of head units; the rest write g and beta
 };
 
-__global__ __launch_bounds__(kPrepThreadsDn) void k_deltanet_prep(DnPrepArgs a) {
-  const int rs = blockIdx.x;  // b * t + s
-  const int b = rs / a.t, s = rs - b * a.t;
-  const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
-  const int k1 = a.conv_k - 1;
-  const int C = 2 * a.kh * a.kd + a.vh * a.vd;
-  const int64_t slot = a.slot[b];
-  const bool slot_ok = slot >= 0 && slot < a.slots_total;
-  const int units = 2 * a.kh + a.vh;
-  const int u = blockIdx.y * (kPrepThreadsDn / kWave) + wave;
-  if (u < units) {
-    const bool is_v = u >= 2 * a.kh;
-    const int dim = is_v ? a.vd : a.kd;
-    const int c0 = is_v ? 2 * a.kh * a.kd + (u - 2 * a.kh) * a.vd : u * a.kd;
-    float x[kPrepMaxPerLane];
-    float ss = 0.f;
-#pragma unroll
-    for (int i = 0; i < kPrepMaxPerLane; ++i) {
-      const int ch = lane + kWave * i;
-      x[i] = 0.f;
-      if (ch >= dim) continue;
-      const int c = c0 + ch;
-      float acc = 0.f;
-#pragma unroll
-      for (int j = 0; j < kConvMaxK1 + 1; ++j) {  // all taps' loads issued together
-        if (j >= a.conv_k) break;
-        const int p = s + j;  // window column: the stored k1, then the t new ones
-        const float win = p < k1 ? (slot_ok ? load_float(a.conv, a.dt, (slot * C + c) * k1 + p) : 0.f)
-                                 : load_float(a.proj, a.dt, ((int64_t)b * a.t + p - k1) * a.proj_stride + c);
-        const float prod = __fmul_rn(win, load_float(a.conv_w, a.dt, (int64_t)c * a.conv_k + j));
-        acc = j == 0 ? prod : __fadd_rn(acc, prod);
-      }
-      float y = acc / (1.f + expf(-acc));
-      if (a.dt == MTPK_BF16) y = bf16_to_f32(f32_to_bf16(y));
-      x[i] = y;
-      ss += y * y;
-    }
-    if (is_v) {
-      float* dst = a.v + ((int64_t)rs * a.vh + (u - 2 * a.kh)) * a.vd;
-#pragma unroll
-      for (int i = 0; i < kPrepMaxPerLane; ++i)
-        if (lane + kWave * i < dim) dst[lane + kWave * i] = x[i];
-    } else {
-      const bool is_q = u < a.kh;
-      const float inv = rsqrtf(wave_sum(ss) + a.eps);
-      const float sc = is_q ? a.q_scale : 1.f;
-      float* dst = (is_q ? a.q : a.k) + ((int64_t)rs * a.kh + (is_q ? u : u - a.kh)) * a.kd;
-#pragma unroll
-      for (int i = 0; i < kPrepMaxPerLane; ++i)
-        if (lane + kWave * i < dim) dst[lane + kWave * i] = x[i] * inv * sc;
-    }
+// Channels ch, ch + 1 of one raw column (`two`: both exist). PAIR: bf16, one dword.
+template <bool PAIR>
+__device__ inline float2 dn_column(const void* p, int dt, int64_t i, bool two) {
+  if (PAIR) {
+    const uint32_t d = *reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(p) + i);
+    return make_float2(bits_f32(d << 16), bits_f32(d & 0xffff0000u));
   }
-  for (int h = tid; blockIdx.y == 0 && h < a.vh; h += kPrepThreadsDn) {
-    const int64_t base = (int64_t)rs * a.proj_stride + C + a.vh * a.vd;
+  return make_float2(load_float(p, dt, i), two ? load_float(p, dt, i + 1) : 0.f);
+}
+
+// K: conv_k when known at compile time, else 0. PAIR: bf16 with an even proj_stride and even head
+// dims, so that every channel pair is a 4-byte aligned dword (its 4 taps 16 bytes, aligned). NI: 128-channel parts of a head.
+template <int K, bool PAIR, int NI, int R>
+__global__ __launch_bounds__(kPrepThreadsDn) void k_deltanet_prep(DnPrepArgs a) {
+  const int tid = threadIdx.x, wave = uniform(tid / kWave), lane = tid & (kWave - 1);
+  const int C = 2 * a.kh * a.kd + a.vh * a.vd;
+  if ((int)blockIdx.x >= a.unit_blocks) {
+    const int64_t i = ((int64_t)blockIdx.x - a.unit_blocks) * kPrepThreadsDn + tid;
+    if (i >= (int64_t)a.B * a.t * a.vh) return;
+    const int64_t rs = i / a.vh;
+    const int h = (int)(i - rs * a.vh);
+    const int64_t base = rs * a.proj_stride + C + a.vh * a.vd;
     const float braw = load_float(a.proj, a.dt, base + h);
     const float araw = load_float(a.proj, a.dt, base + a.vh + h);
     const float x = __fadd_rn(araw, a.dt_bias[h]);
     const float sp = x > 20.f ? x : log1pf(expf(x));
-    a.beta[(int64_t)rs * a.vh + h] = 1.f / (1.f + expf(-braw));
-    a.g[(int64_t)rs * a.vh + h] = -expf(a.a_log[h]) * sp;
+    a.beta[i] = 1.f / (1.f + expf(-braw));
+    a.g[i] = -expf(a.a_log[h]) * sp;
+    return;
   }
+  const int conv_k = K ? K : a.conv_k, k1 = conv_k - 1;
+  constexpr int KM = K ? K : kConvMaxK1 + 1;
+  const int units = 2 * a.kh + a.vh, runs = (a.t + R - 1) / R;
+  const int64_t id = (int64_t)blockIdx.x * (kPrepThreadsDn / kWave) + wave;
+  const int u = (int)(id % units);
+  const int64_t br = id / units;
+  if (br >= (int64_t)a.B * runs) return;
+  const int b = (int)(br / runs), s0 = (int)(br - (int64_t)b * runs) * R;
+  const int rows = min(R, a.t - s0);
+  const int64_t slot = a.slot[b];
+  const bool slot_ok = slot >= 0 && slot < a.slots_total;
+  const bool is_v = u >= 2 * a.kh;
+  const int dim = is_v ? a.vd : a.kd;
+  const int c0 = is_v ? 2 * a.kh * a.kd + (u - 2 * a.kh) * a.vd : u * a.kd;
+  const int64_t row0 = (int64_t)b * a.t;
+  float2 x[NI][R];
+  float ss[R];
+#pragma unroll
+  for (int s = 0; s < R; ++s) ss[s] = 0.f;
+#pragma unroll
+  for (int n = 0; n < NI; ++n) {
+    const int ch = 2 * lane + 128 * n;
+    const bool one = ch < dim, two = ch + 1 < dim;
+    const int c = c0 + (one ? ch : 0);
+    // columns s0 - k1 .. s0 + R - 1 of [the stored window | the new columns]; entry j is column
+    // s0 - k1 + j, and rows past the last one repeat it
+    float2 win[R + KM - 1], w[KM];
+#pragma unroll
+    for (int j = 0; j < R + KM - 1; ++j) {
+      const int p = s0 + j - k1;
+      win[j] = make_float2(0.f, 0.f);
+      if (j >= R + k1) continue;
+      if (j >= k1 || p >= 0)  // the first rows' window columns come from the state below
+        win[j] = dn_column<PAIR>(a.proj, a.dt, (row0 + min(p, a.t - 1)) * a.proj_stride + c, two);
+    }
+    if (s0 < k1 && slot_ok) {  // s0 == 0, or every row of a short call: entries j < k1 - s0
+      const int64_t i = (slot * C + c) * k1;
+      if (PAIR && K == 4) {  // two channels of 3 columns: 12 bytes
+        const uint32_t* const d = reinterpret_cast<const uint32_t*>(static_cast<const uint16_t*>(a.conv) + i);
+        const uint32_t d0 = d[0], d1 = d[1], d2 = d[2];
+        win[0] = make_float2(bits_f32(d0 << 16), bits_f32(d1 & 0xffff0000u));
+        win[1] = make_float2(bits_f32(d0 & 0xffff0000u), bits_f32(d2 << 16));
+        win[2] = make_float2(bits_f32(d1 << 16), bits_f32(d2 & 0xffff0000u));
+      } else {
+#pragma unroll
+        for (int j = 0; j < KM - 1; ++j)
+          if (j < k1 - s0)
+            win[j] = make_float2(load_float(a.conv, a.dt, i + s0 + j), two ? load_float(a.conv, a.dt, i + k1 + s0 + j) : 0.f);
+      }
+    }
+    if (PAIR && K == 4) {  // two channels of 4 taps: 16 bytes
+      const u32x4_t d = ld16(static_cast<const uint16_t*>(a.conv_w) + (int64_t)c * 4);
+      w[0] = make_float2(bits_f32(d[0] << 16), bits_f32(d[2] << 16));
+      w[1] = make_float2(bits_f32(d[0] & 0xffff0000u), bits_f32(d[2] & 0xffff0000u));
+      w[2] = make_float2(bits_f32(d[1] << 16), bits_f32(d[3] << 16));
+      w[3] = make_float2(bits_f32(d[1] & 0xffff0000u), bits_f32(d[3] & 0xffff0000u));
+    } else {
+#pragma unroll
+      for (int j = 0; j < KM; ++j) {
+        const int64_t i = (int64_t)c * conv_k + j;
+        w[j] = make_float2(0.f, 0.f);
+        if (j < conv_k)
+          w[j] = make_float2(load_float(a.conv_w, a.dt, i), two ? load_float(a.conv_w, a.dt, i + conv_k) : 0.f);
+      }
+    }
+#pragma unroll
+    for (int s = 0; s < R; ++s) {
+      float acc[2] = {0.f, 0.f};
+#pragma unroll
+      for (int j = 0; j < KM; ++j) {
+        const float p0 = __fmul_rn(win[s + j].x, w[j].x), p1 = __fmul_rn(win[s + j].y, w[j].y);
+        if (j < conv_k) {
+          acc[0] = j == 0 ? p0 : __fadd_rn(acc[0], p0);
+          acc[1] = j == 0 ? p1 : __fadd_rn(acc[1], p1);
+        }
+      }
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        float y = acc[e] / (1.f + expf(-acc[e]));
+        if (a.dt == MTPK_BF16) y = bf16_to_f32(f32_to_bf16(y));
+        if (!(e ? two : one)) y = 0.f;
+        (e ? x[n][s].y : x[n][s].x) = y;
+        ss[s] += y * y;
+      }
+    }
+  }
+  float* dst;
+  int64_t step;
+  if (is_v) {
+    dst = a.v + ((row0 + s0) * a.vh + (u - 2 * a.kh)) * a.vd;
+    step = (int64_t)a.vh * a.vd;
+  } else {
+    const bool is_q = u < a.kh;
+    dst = (is_q ? a.q : a.k) + ((row0 + s0) * a.kh + (is_q ? u : u - a.kh)) * a.kd;
+    step = (int64_t)a.kh * a.kd;
+    const float sc = is_q ? a.q_scale : 1.f;
+#pragma unroll
+    for (int s = 0; s < R; ++s) {
+      const float inv = rsqrtf(wave_sum(ss[s]) + a.eps);
+#pragma unroll
+      for (int n = 0; n < NI; ++n) x[n][s] = make_float2(x[n][s].x * inv * sc, x[n][s].y * inv * sc);
+    }
+  }
+#pragma unroll
+  for (int s = 0; s < R; ++s) {
+    if (s >= rows) continue;
+#pragma unroll
+    for (int n = 0; n < NI; ++n) {
+      const int ch = 2 * lane + 128 * n;
+      float* const o = dst + s * step + ch;
+      if (PAIR) {  // even dims: an 8-byte aligned pair
+        if (ch < dim) *reinterpret_cast<float2*>(o) = x[n][s];
+      } else {
+        if (ch < dim) o[0] = x[n][s].x;
+        if (ch + 1 < dim) o[1] = x[n][s].y;
+      }
+    }
+  }
+}
+
+template <int K, bool PAIR, int NI>
+int launch_deltanet_prep(DnPrepArgs a, hipStream_t st) {
+  const int R = a.t <= 4 ? 4 : kPrepRows;
+  const int64_t waves = (int64_t)a.B * ((a.t + R - 1) / R) * (2 * a.kh + a.vh);
+  const int64_t ub = (waves + kPrepThreadsDn / kWave - 1) / (kPrepThreadsDn / kWave);
+  const int64_t gb = ((int64_t)a.B * a.t * a.vh + kPrepThreadsDn - 1) / kPrepThreadsDn;
+  if (ub + gb > INT32_MAX) return MTPK_EINVAL;
+  a.unit_blocks = (int)ub;
+  auto kern = R == 4 ? k_deltanet_prep<K, PAIR, NI, 4> : k_deltanet_prep<K, PAIR, NI, kPrepRows>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(ub + gb)), dim3(kPrepThreadsDn), 0, st, a);
+  return status_of(hipGetLastError());
 }
 
 // The commit's conv-window update (`deltanet_verify_rollback`, model.py:3907-3972): slot b's
@@ -604,20 +709,24 @@ int mtpk_deltanet_prep(const void* proj, int dtype, int64_t proj_stride, const v
   if (batch < 0 || t < 1 || k_heads < 1 || v_heads < 1 || conv_k < 2 || conv_k > kConvMaxK1 + 1 ||
       slots_total < 1)
     return MTPK_EINVAL;
-  if (k_dim < 1 || k_dim > kWave * kPrepMaxPerLane || v_dim < 1 || v_dim > kWave * kPrepMaxPerLane)
-    return MTPK_EINVAL;
+  if (k_dim < 1 || k_dim > kPrepMaxDim || v_dim < 1 || v_dim > kPrepMaxDim) return MTPK_EINVAL;
   const int64_t C = 2 * k_heads * k_dim + v_heads * v_dim;
   if (proj_stride < C + v_heads * v_dim + 2 * v_heads || batch * t > INT32_MAX) return MTPK_EINVAL;
+  // head units of one row: at most 262140
+  if ((2 * k_heads + v_heads + 3) / 4 > 65535) return MTPK_EINVAL;
   if (batch == 0) return 0;
-  DnPrepArgs a{proj, proj_stride, conv_state, slot, slots_total, conv_w, a_log, dt_bias, dtype, (int)t,
-               (int)k_heads, (int)k_dim, (int)v_heads, (int)v_dim, (int)conv_k, eps, q_scale,
-               q, k, v, g, beta};
-  const int64_t units = 2 * k_heads + v_heads;
-  const int64_t groups = (units + kPrepThreadsDn / kWave - 1) / (kPrepThreadsDn / kWave);
-  if (groups > 65535) return MTPK_EINVAL;
-  hipLaunchKernelGGL(k_deltanet_prep, dim3((unsigned)(batch * t), (unsigned)groups),
-                     dim3(kPrepThreadsDn), 0, (hipStream_t)stream, a);
-  return status_of(hipGetLastError());
+  const DnPrepArgs a{proj, proj_stride, conv_state, slot, slots_total, conv_w, a_log, dt_bias, (int)batch,
+                     dtype, (int)t, (int)k_heads, (int)k_dim, (int)v_heads, (int)v_dim, (int)conv_k, eps,
+                     q_scale, q, k, v, g, beta, 0};
+  const hipStream_t st = (hipStream_t)stream;
+  auto at8 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 7u) == 0; };
+  const bool pair = dtype == MTPK_BF16 && proj_stride % 2 == 0 && k_dim % 2 == 0 && v_dim % 2 == 0 &&
+                    ((reinterpret_cast<uintptr_t>(proj) | reinterpret_cast<uintptr_t>(conv_state)) & 3u) == 0 &&
+                    aligned16(conv_w) && at8(q) && at8(k) && at8(v);
+  const bool wide = k_dim > 128 || v_dim > 128;
+  if (pair && conv_k == 4)
+    return wide ? launch_deltanet_prep<4, true, 2>(a, st) : launch_deltanet_prep<4, true, 1>(a, st);
+  return launch_deltanet_prep<0, false, 2>(a, st);
 }
 
 int mtpk_conv_commit(void* conv_state, int dtype, const int64_t* slot, int64_t slots_total,

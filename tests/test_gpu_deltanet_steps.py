@@ -15,7 +15,7 @@ import torch
 import deltanet
 from oracle import deltanet_ref as dn
 
-from .test_gpu_deltanet import _case, _dev
+from .test_gpu_deltanet import _case, _dev, _torch_prep
 
 pytestmark = pytest.mark.gpu
 
@@ -118,3 +118,28 @@ def test_long_commit_is_the_rule_and_the_window(dev) -> None:
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(p1, p3) and torch.equal(c1, c3)
+
+
+@pytest.mark.parametrize("dtype,t,conv_k,kd,vd", [
+    (torch.bfloat16, 4, 4, 128, 128), (torch.bfloat16, 5, 4, 64, 128),  # 4 rows a wave, then 8
+    (torch.bfloat16, 17, 4, 128, 192), (torch.bfloat16, 9, 4, 33, 128), (torch.bfloat16, 8, 2, 128, 20),
+    (torch.bfloat16, 25, 9, 128, 128), (torch.float32, 11, 4, 16, 256), (torch.float32, 3, 6, 130, 7),
+])
+def test_prep_runs_of_rows(dev, dtype, t, conv_k, kd, vd) -> None:
+    """`deltanet.prep` at the edges of its runs of rows, odd head dims and other windows, against the
+    torch chain: sums in the same order, so f32 within a few roundings, and bf16 within the
+    neighbouring value where a SiLU lies at a tie."""
+    g = torch.Generator().manual_seed(t)
+    b, kh, vh = 2, 2, 4
+    c = 2 * kh * kd + vh * vd
+    proj = (torch.randn(b, t, c + vh * vd + 2 * vh, generator=g) * 2).to(dtype).to(dev)
+    conv = torch.randn(3, c, conv_k - 1, generator=g).to(dtype).to(dev)
+    w = (torch.randn(c, conv_k, generator=g) * 0.3).to(dtype).to(dev)
+    a_log, bias = torch.rand(vh, generator=g).to(dev), torch.rand(vh, generator=g).to(dev)
+    slots = torch.tensor([2, 0], device=dev)
+    got = deltanet.prep(proj, conv, slots, w, a_log, bias, kh, kd, vh, vd)
+    want = _torch_prep(proj, conv, slots, w, a_log, bias, kh, kd, vh, vd)
+    for x, y in zip(got, want, strict=True):
+        tol = 2**-7 if dtype == torch.bfloat16 else 1e-5
+        torch.testing.assert_close(x, y, rtol=tol, atol=1e-6)
+        assert float(((x - y).abs() > 1e-5 * y.abs() + 1e-6).float().mean()) < 2e-3
