@@ -31,8 +31,14 @@ MTPK_HD float bits_f32(uint32_t u) {
   return v.f;
 }
 
-// fp32 -> bf16, round to nearest even. NaN stays a quiet NaN.
+// fp32 -> bf16, round to nearest even. NaN stays a quiet NaN. On the device this is gfx950's own
+// conversion (one instruction for one or two values; the integer form is six and a branch around
+// the NaN, which made the rounding the largest part of several epilogues); the bits agree for every
+// input but a NaN's payload.
 MTPK_HD uint16_t f32_to_bf16(float f) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_bit_cast(uint16_t, (__bf16)f);
+#endif
   uint32_t u = f32_bits(f);
   if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40u);
   u += 0x7fffu + ((u >> 16) & 1u);

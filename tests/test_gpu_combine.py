@@ -123,3 +123,22 @@ def test_bw_prep_partitions_the_live_assignments(dev, tokens):
         seen += ids
     assert sorted(seen) == live
     assert n <= plan.u_max
+
+
+def test_bf16_rounding_of_every_kind_of_value(dev) -> None:
+    """The rounding that stores use, through a one-row combine, against torch's on the CPU bit for
+    bit: every exponent, ties both ways, denormals, the overflow to infinity, infinities, NaN."""
+    g = torch.Generator().manual_seed(0)
+    bits = torch.randint(-(2**31), 2**31, (1 << 20,), generator=g, dtype=torch.int64).to(torch.int32)
+    top = torch.arange(1 << 16, dtype=torch.int32) << 16  # every bf16 and the ties around it
+    bits = torch.cat([bits, top, top | 0x8000, top | 0x7FFF, top | 0x8001])
+    y = bits.view(torch.float32).reshape(-1, 4096)
+    rows = y.shape[0]
+    out = torch.empty(rows, 4096, dtype=torch.bfloat16, device=dev)
+    mxfp4_gemv.bw_combine(y.to(dev), torch.zeros(rows, dtype=torch.int32, device=dev),
+                          torch.ones(rows, device=dev), (0, 1), 1, out)
+    want = (y + 0.0).bfloat16()
+    got = out.cpu()
+    assert torch.equal(got.isnan(), want.isnan())
+    ok = ~want.isnan()
+    assert torch.equal(got.view(torch.int16)[ok], want.view(torch.int16)[ok])
