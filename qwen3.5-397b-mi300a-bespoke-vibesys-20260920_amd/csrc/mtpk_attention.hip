@@ -95,12 +95,21 @@ struct AttnIO {
   AttnRows gr;
 };
 
-__device__ inline uint16_t attn_out_value(const AttnIO& io, float v, int b, int h, int s, int d) {
-  if (!io.gate) return f32_to_bf16(v);
-  const float g = bf16_to_f32(io.gate[io.gr.at(b, h, s) + d]);
-  const float sg = bf16_to_f32(f32_to_bf16(1.f / (1.f + expf(-g))));
+__device__ inline uint16_t attn_gated(bool gated, uint16_t gate, float v) {
+  if (!gated) return f32_to_bf16(v);
+  const float sg = bf16_to_f32(f32_to_bf16(1.f / (1.f + expf(-bf16_to_f32(gate)))));
   return f32_to_bf16(bf16_to_f32(f32_to_bf16(v)) * sg);
 }
+
+__device__ inline uint16_t attn_out_value(const AttnIO& io, float v, int b, int h, int s, int d) {
+  return attn_gated(io.gate != nullptr, io.gate ? io.gate[io.gr.at(b, h, s) + d] : (uint16_t)0, v);
+}
+
+}  // namespace mtpk
+
+#include "mtpk_attention_prompt.h"
+
+namespace mtpk {
 
 template <int HD>
 __global__ __launch_bounds__(kAttnThreads) void k_paged_attention(
@@ -295,61 +304,99 @@ __global__ __launch_bounds__(kAttnThreads) void k_paged_attention(
 }
 
 // Merge of the key splits: out = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M), M = max_s m_s,
-// over the splits that hold keys of the row's lane. One thread per (row, 4 d values).
-template <int HD>
+// over the splits that hold keys of the row. W waves per row: each weighs all splits at once (lane
+// s split s, at most 64), then takes every W-th split, HD / 64 adjacent values a lane, four splits'
+// loads in flight; the waves' sums are added in order. A row then waits for three memory latencies
+// whatever the split count (a thread per 4 values that walked the splits twice took 39 us for 96
+// rows of 64 splits; this 7 us). W = 1, four rows to a workgroup, up to 8 splits, where the rows
+// themselves fill the chip (6144 rows of 5 splits: 20 us with W = 4).
+constexpr int kMergeSplits = 64;
+
+template <int HD, bool PROMPT, int W>
 __global__ __launch_bounds__(256) void k_attention_merge(
     const float* __restrict__ part_o, const float* __restrict__ part_ml,
-    const int64_t* __restrict__ base_pos, int B, int t, int heads, int kvh, int n_split,
+    const int64_t* __restrict__ base_pos, int rows, int t, int heads, int kvh, int n_split,
     int row_groups, AttnIO io) {
+  constexpr int NV = HD / kWave;  // values per lane
+  typedef float vec_t __attribute__((ext_vector_type(NV)));
+  __shared__ vec_t red[W][kWave];
   const int group = heads / kvh;
-  const int64_t rows = (int64_t)B * heads * t;
-  const int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= rows * (HD / 4)) return;
-  const int64_t row = idx / (HD / 4);
-  const int d = (int)(idx % (HD / 4)) * 4;
-  const int st = (int)(row % t);
-  const int64_t bh = row / t;
-  const int hq = (int)(bh % heads), b = (int)(bh / heads);
-  const int kh = hq / group, r = (hq % group) * t + st;
-  const int rg = r / kAttnRows, rl = r % kAttnRows;
-  const int ctx = (int)base_pos[b] + t;
-  const int64_t base = ((int64_t)(b * kvh + kh) * row_groups + rg) * n_split;
-  float mx = -INFINITY;
-  for (int sp = 0; sp < n_split; ++sp) {
-    int k0, k1;
-    attn_split_range(ctx, n_split, sp, k0, k1);
-    if (k0 < k1) mx = fmaxf(mx, part_ml[((base + sp) * kAttnRows + rl) * 2]);
-  }
-  float lsum = 0.f, acc[4] = {0.f, 0.f, 0.f, 0.f};
-  for (int sp = 0; sp < n_split; ++sp) {
-    int k0, k1;
-    attn_split_range(ctx, n_split, sp, k0, k1);
-    if (k0 >= k1) continue;
-    const int64_t pr = (base + sp) * kAttnRows + rl;
-    const float ms = part_ml[pr * 2];
-    const float w = ms == -INFINITY ? 0.f : exp2f(ms - mx);
-    lsum += part_ml[pr * 2 + 1] * w;
-    const float* po = part_o + pr * HD + d;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = W == 1 ? 0 : uniform(tid / kWave);
+  const int row = W == 1 ? uniform((int)blockIdx.x * 4 + tid / kWave) : (int)blockIdx.x;
+  if (row >= rows) return;  // uniform over the wave (W == 1: no barrier below)
+  const int st = row % t, bh = row / t, hq = bh % heads, b = bh / heads, kh = hq / group;
+  const int r = PROMPT ? st * group + hq % group : (hq % group) * t + st;
+  constexpr int kRows = PROMPT ? kPromptRows : kAttnRows;
+  const int rg = r / kRows, rl = r % kRows;
+  const int bp = (int)base_pos[b];
+  const int ctx = PROMPT ? prompt_keys_end(bp, rg, group * t, group) : bp + t;
+  const int64_t base = (((int64_t)(b * kvh + kh) * row_groups + rg) * n_split) * kRows + rl;
+  int k0, k1;
+  attn_split_range(ctx, n_split, lane, k0, k1);
+  const bool live = lane < n_split && k0 < k1;
+  const float ml = live ? part_ml[(base + (int64_t)lane * kRows) * 2] : -INFINITY;
+  const float ll = live ? part_ml[(base + (int64_t)lane * kRows) * 2 + 1] : 0.f;
+  const float mx = wave_max(ml);
+  const float w = ml == -INFINITY ? 0.f : exp2f(ml - mx);
+  const float inv = 1.f / wave_sum(ll * w);
+  vec_t acc = {};
+  for (int s0 = wave; s0 < n_split; s0 += 4 * W) {
+    vec_t v[4];
+    float ws[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] += po[e] * w;
-  }
-  const float inv = 1.f / lsum;
-  uint16_t* orow = io.out + io.orow.at(b, hq, st) + d;
+    for (int i = 0; i < 4; ++i) {
+      const int s = s0 + W * i;
+      ws[i] = s < n_split ? __shfl(w, s & (kWave - 1), kWave) : 0.f;  // 0 for a split without keys
+      v[i] = vec_t{};
+      if (ws[i] != 0.f) v[i] = *reinterpret_cast<const vec_t*>(part_o + (base + (int64_t)s * kRows) * HD + NV * lane);
+    }
 #pragma unroll
-  for (int e = 0; e < 4; ++e) orow[e] = attn_out_value(io, acc[e] * inv, b, hq, st, d + e);
+    for (int i = 0; i < 4; ++i) acc += v[i] * ws[i];
+  }
+  if (W > 1) {
+    red[wave][lane] = acc;
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int i = 1; i < W; ++i) acc += red[i][lane];
+  }
+  uint16_t* const orow = io.out + io.orow.at(b, hq, st) + NV * lane;
+#pragma unroll
+  for (int e = 0; e < NV; ++e) orow[e] = attn_out_value(io, acc[e] * inv, b, hq, st, NV * lane + e);
 }
 
-// Workgroups of k_paged_attention<HD> resident on the whole device at once.
-int attention_slots(int hd) {
-  static int occ[3] = {0, 0, 0};
-  const int i = hd == 64 ? 0 : hd == 128 ? 1 : 2;
+// Workgroups of the attention kernel for head dim `hd` (the prompt form or not) resident on the
+// whole device at once.
+int attention_slots(int hd, bool prompt) {
+  static int occ[6] = {0, 0, 0, 0, 0, 0};
+  const int i = (hd == 64 ? 0 : hd == 128 ? 1 : 2) + (prompt ? 3 : 0);
   if (occ[i] == 0) {
-    occ[i] = hd == 64    ? occupancy_per_cu(k_paged_attention<64>, kAttnThreads)
-             : hd == 128 ? occupancy_per_cu(k_paged_attention<128>, kAttnThreads)
-                         : occupancy_per_cu(k_paged_attention<256>, kAttnThreads);
+    switch (i) {
+      case 0: occ[i] = occupancy_per_cu(k_paged_attention<64>, kAttnThreads); break;
+      case 1: occ[i] = occupancy_per_cu(k_paged_attention<128>, kAttnThreads); break;
+      case 2: occ[i] = occupancy_per_cu(k_paged_attention<256>, kAttnThreads); break;
+      case 3: occ[i] = occupancy_per_cu(k_prompt_attention<64>, 256); break;
+      case 4: occ[i] = occupancy_per_cu(k_prompt_attention<128>, 256); break;
+      default: occ[i] = occupancy_per_cu(k_prompt_attention<256>, 256); break;
+    }
     if (occ[i] < 1) occ[i] = 1;
   }
   return device_cu_count() * occ[i];
+}
+
+// Rows per kv head from which a call takes the prompt form, one whole workgroup's: below, part of it
+// would be empty, and verify rounds (64 to 80 rows) read long contexts that the decode form streams.
+// 125 rows of 32 heads of 128: 18.7 against 19.5 us; 100 rows of 256 over 1500 cached keys: 33
+// against 40 us; 2047 rows: 98 against 392 us.
+constexpr int64_t kPromptMinRows = 128;
+bool attention_prompt(int64_t rows) { return rows >= kPromptMinRows; }
+int64_t attention_row_groups(int64_t rows);
+int64_t attention_part_rows(int64_t rows) {  // rows of a (lane, kv head)'s partial results, padded
+  return attention_row_groups(rows) * (attention_prompt(rows) ? kPromptRows : kAttnRows);
+}
+int64_t attention_row_groups(int64_t rows) {
+  const int64_t per = attention_prompt(rows) ? kPromptRows : kAttnRows;
+  return (rows + per - 1) / per;
 }
 
 // The largest key-split count whose workgroups all run in one round of resident slots, at
@@ -357,13 +404,13 @@ int attention_slots(int hd) {
 // for its whole length, and every extra split adds partials to the merge: at 48 lanes, 2 kv
 // heads of 256 and 8192 keys (96 workgroups per split, 512 slots), 5 splits take 179 us per
 // call against 199 us for 8 and 10 and 220 us for 12 and 16.
-int attention_splits(int hd, int64_t B, int64_t kvh, int row_groups, int64_t max_ctx) {
-  const int64_t wgs = B * kvh * row_groups;
-  const int64_t fit = attention_slots(hd) / (wgs > 0 ? wgs : 1);
+int attention_splits(int hd, int64_t B, int64_t kvh, int64_t rows, int64_t max_ctx) {
+  const int64_t wgs = B * kvh * attention_row_groups(rows);
+  const int64_t fit = attention_slots(hd, attention_prompt(rows)) / (wgs > 0 ? wgs : 1);
   const int64_t tiles = (max_ctx + kAttnKeys - 1) / kAttnKeys;
   const int64_t cap = tiles / 8 > 1 ? tiles / 8 : 1;  // at least 8 tiles per split
   int64_t n = fit < cap ? fit : cap;
-  if (n > 64) n = 64;
+  if (n > kMergeSplits) n = kMergeSplits;
   return n < 1 ? 1 : (int)n;
 }
 
@@ -372,16 +419,31 @@ int launch_attention(const AttnIO& io, const uint16_t* k_pool, const uint16_t* v
                      int64_t pool_rows, const int32_t* table, int table_stride,
                      const int64_t* base_pos, int B, int t, int heads, int kvh, float scale,
                      int n_split, float* part_o, float* part_ml, hipStream_t st) {
-  const int row_groups = (heads / kvh * t + kAttnRows - 1) / kAttnRows;
+  const int64_t rows = (int64_t)(heads / kvh) * t;
+  const bool prompt = attention_prompt(rows);
+  const int row_groups = (int)attention_row_groups(rows);
   const float scale_log2 = scale * 1.4426950408889634f;
-  hipLaunchKernelGGL(k_paged_attention<HD>, dim3(B * kvh * row_groups, n_split), dim3(kAttnThreads),
-                     0, st, io, k_pool, v_pool, pool_rows, table, table_stride, base_pos, t, heads,
-                     kvh, scale_log2, n_split, row_groups, part_o, part_ml);
+  const int64_t grid = (int64_t)B * kvh * row_groups;
+  if (prompt) {
+    auto on16 = [](const void* p, const AttnRows& r) { return aligned16(p) && ((r.sb | r.sh | r.st) & 7) == 0; };
+    const int wide = on16(io.out, io.orow) && (!io.gate || on16(io.gate, io.gr));
+    const int paired = n_split == 1 && grid > device_cu_count() && grid <= attention_slots(HD, true);
+    hipLaunchKernelGGL(k_prompt_attention<HD>, dim3((unsigned)grid, n_split), dim3(256), 0, st, io, k_pool,
+                       v_pool, pool_rows, table, table_stride, base_pos, t, heads, kvh, B * kvh, scale_log2,
+                       n_split, row_groups, paired, wide, part_o, part_ml);
+  } else {
+    hipLaunchKernelGGL(k_paged_attention<HD>, dim3((unsigned)grid, n_split), dim3(kAttnThreads), 0, st, io,
+                       k_pool, v_pool, pool_rows, table, table_stride, base_pos, t, heads, kvh, scale_log2,
+                       n_split, row_groups, part_o, part_ml);
+  }
   int rc = status_of(hipGetLastError());
   if (rc || n_split == 1) return rc;
-  const int64_t threads = (int64_t)B * heads * t * (HD / 4);
-  hipLaunchKernelGGL(k_attention_merge<HD>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st,
-                     part_o, part_ml, base_pos, B, t, heads, kvh, n_split, row_groups, io);
+  const int out_rows = B * heads * t;
+  const bool few = n_split <= 8;
+  auto merge = prompt ? (few ? k_attention_merge<HD, true, 1> : k_attention_merge<HD, true, 4>)
+                      : (few ? k_attention_merge<HD, false, 1> : k_attention_merge<HD, false, 4>);
+  hipLaunchKernelGGL(merge, dim3((unsigned)(few ? (out_rows + 3) / 4 : out_rows)), dim3(256), 0, st, part_o,
+                     part_ml, base_pos, out_rows, t, heads, kvh, n_split, row_groups, io);
   return status_of(hipGetLastError());
 }
 
@@ -435,16 +497,13 @@ int mtpk_attention_splits(int64_t batch, int64_t t, int64_t heads, int64_t kv_he
                           int64_t head_dim, int64_t max_ctx) {
   if (batch <= 0 || t <= 0 || kv_heads <= 0 || heads % kv_heads) return 0;
   if (head_dim != 64 && head_dim != 128 && head_dim != 256) return 0;
-  const int row_groups = (int)((heads / kv_heads * t + kAttnRows - 1) / kAttnRows);
-  return attention_splits((int)head_dim, batch, kv_heads, row_groups, max_ctx);
+  return attention_splits((int)head_dim, batch, kv_heads, heads / kv_heads * t, max_ctx);
 }
 
 int64_t mtpk_attention_workspace_bytes(int64_t batch, int64_t t, int64_t heads, int64_t kv_heads,
                                        int64_t head_dim, int n_split) {
   if (batch <= 0 || t <= 0 || kv_heads <= 0 || heads % kv_heads || n_split <= 1) return 0;
-  const int64_t row_groups = (heads / kv_heads * t + kAttnRows - 1) / kAttnRows;
-  const int64_t slots = batch * kv_heads * row_groups * n_split * kAttnRows;
-  return slots * (head_dim + 2) * 4;
+  return batch * kv_heads * attention_part_rows(heads / kv_heads * t) * n_split * (head_dim + 2) * 4;
 }
 
 namespace {
@@ -468,9 +527,9 @@ int paged_attention_io(const AttnIO& io, int64_t batch, int64_t t, int64_t heads
                                                                       head_dim, n_split)))
     return MTPK_EINVAL;
   if (batch == 0) return 0;
-  const int64_t rg = (heads / kv_heads * t + kAttnRows - 1) / kAttnRows;
   float* part_o = (float*)workspace;
-  float* part_ml = part_o ? part_o + batch * kv_heads * rg * n_split * kAttnRows * head_dim : nullptr;
+  float* part_ml = part_o ? part_o + batch * kv_heads * attention_part_rows(heads / kv_heads * t) * n_split * head_dim
+                          : nullptr;
   const hipStream_t st = (hipStream_t)stream;
 #define MTPK_ATTN(HD_)                                                                          \
   launch_attention<HD_>(io, k_pool, v_pool, pool_rows, block_table, (int)table_stride, base_pos, \
