@@ -9,6 +9,7 @@
 //               as bf16 hi/lo planes (16 significant bits)
 //     down      per (unit, 64 hidden rows): same decode, MFMA over both planes; fp32 y
 //     combine   per token: sum of weight * y over its top_k assignments in j order
+//     From 14 assignments per expert the units hold up to 64 tokens (mtpk_moe_wide.h).
 //   direct path (tokens <= 4): gate_up with one unit per assignment (no prep), then a
 //     per-token down that also combines (no y, no combine launch)
 // Each wave keeps a ring of trips (weight + activation loads) in flight ahead of the MFMAs.
@@ -16,6 +17,7 @@
 // Lane mapping and K coverage of one MFMA tile: see mtpk_common.h ("MoE lane mapping").
 
 #include <mutex>
+#include <type_traits>
 
 #include "mtpk_device.h"
 #include "mtpk_gemm_tile.h"
@@ -43,7 +45,7 @@ struct PrepSmem {
 // then reloads the routing only past them.
 constexpr int kPrepKeep = 4;
 
-template <int NT>
+template <int NT, int kUnitTokens = mtpk::kUnitTokens, int kPrepKeep = mtpk::kPrepKeep>
 __device__ inline void prep_body(const void* __restrict__ a_expert, int edt,
                                  const void* __restrict__ a_weight, int wdt, int assignments,
                                  int lo, int n_experts, int32_t* __restrict__ sorted,
@@ -1397,6 +1399,22 @@ __global__ __launch_bounds__(kMoeThreads) void k_moe_down_lds(
   flush_y();
 }
 
+#include "mtpk_moe_wide.h"
+
+// The prep of wide units. One workgroup sorts a prompt's routing, and with few assignments kept it
+// waited for memory once per 1024 of them and pass: a thread loads 24 at once (2048 rows of 10:
+// 35 -> 29 us).
+constexpr int kPrepWideKeep = 24;
+__global__ __launch_bounds__(kPrepThreads) void k_moe_prep_wide(
+    const void* __restrict__ a_expert, int edt, const void* __restrict__ a_weight, int wdt,
+    int assignments, int lo, int n_experts, int32_t* __restrict__ sorted,
+    int32_t* __restrict__ units, int max_units, int32_t* __restrict__ n_units) {
+  __shared__ __attribute__((aligned(16))) uint8_t smem[PrepSmem<kPrepThreads>::kBytes];
+  prep_body<kPrepThreads, kWideTokens, kPrepWideKeep>(a_expert, edt, a_weight, wdt, assignments, lo,
+                                                      n_experts, sorted, units, max_units, n_units,
+                                                      smem);
+}
+
 // ---------------------------------------------------------------- combine (unit mode)
 //
 // out[t, n..n+3] = sum_j w_j * y[t*top_k + j, n..n+3] over live assignments, in j order. The
@@ -1974,6 +1992,35 @@ UnitSrc unit_direct(const void* a_expert, int edt, const void* a_weight, int wdt
   return s;
 }
 
+// Wide units (mtpk_moe_wide.h): bf16 rows of the LDS kernels' K ranges, offsets below 2^31 (bit 31
+// marks a load that is not made), from kWideMinPerExpert assignments per local expert. Below it most
+// units hold a tile of 16 tokens either way, and the 16-token kernels, with their stores held back
+// and items pipelined, stream weights faster. 512 experts, top-10, Zipf(1.1), 16-token units against
+// wide ones: 256 rows (5 per expert) 539 / 579 us, 400 (8) 660 / 677, 600 (12) 803 / 797, 1024 (20)
+// 1047 / 929, 2048 (40) 1604 / 1259.
+constexpr int64_t kWideMinPerExpert = 14;
+bool wide_units(int64_t tokens, int64_t hidden, int64_t inter_dim, int64_t local_experts, int64_t a) {
+  constexpr int64_t lim = int64_t(1) << 31;
+  return a >= kWideMinPerExpert * local_experts && tokens > kDirectMaxTokens && hidden % 512 == 0 &&
+         hidden <= 4096 && inter_dim % 512 == 0 && inter_dim <= 1024 && tokens * hidden * 2 < lim &&
+         a * inter_dim * 4 < lim;
+}
+
+template <bool UP>
+int launch_wide(const uint16_t* x, int64_t x_elems, int64_t x_plane, int K, const uint8_t* wq,
+                const uint8_t* ws, int N, const UnitSrc& src, int top_k, uint16_t* inter,
+                int64_t inter_plane, float* y, hipStream_t st) {
+  static int occ = 0;
+  auto kern = k_moe_wide<UP>;
+  if (occ == 0) occ = occupancy_per_cu(kern, kWideThreads);
+  constexpr int tiles = UP ? kWideWaves : 4 * kWideWaves;
+  const int64_t items = (int64_t)src.max_units * (((N >> 4) + tiles - 1) / tiles);
+  const int64_t cap = (int64_t)device_cu_count() * occ;
+  hipLaunchKernelGGL(kern, dim3((unsigned)(items < cap ? items : cap)), dim3(kWideThreads), 0, st, x,
+                     (uint32_t)(x_elems * 2), x_plane, K, wq, ws, N, src, top_k, inter, inter_plane, y);
+  return status_of(hipGetLastError());
+}
+
 bool gemm_shapes_ok(int64_t hidden, int64_t inter_dim, int64_t local_experts) {
   return hidden > 0 && hidden % 32 == 0 && inter_dim > 0 && inter_dim % 32 == 0 &&
          hidden <= (1 << 20) && inter_dim <= (1 << 20) && local_experts > 0 &&
@@ -2266,15 +2313,36 @@ int mtpk_fused_moe_shared(const void* x, int x_dtype, int64_t tokens, int64_t hi
                        dim3(256), 0, (hipStream_t)stream, out, x_dtype, (int)hidden, st);
     return status_of(hipGetLastError());
   }
-  rc = mtpk_moe_prep(a_expert, expert_dtype, a_weight, weight_dtype, a, expert_lo, expert_hi,
-                     sorted, units, mu, n_units, stream);
-  if (rc) return rc;
-  rc = mtpk_moe_gate_up(xplanes, xp, tokens, hidden, gate_up, gate_up_scale, local_experts,
-                        inter_dim, sorted, units, n_units, mu, top_k, inter, ip, a, stream);
-  if (rc) return rc;
-  rc = mtpk_moe_down(inter, ip, a, inter_dim, down, down_scale, local_experts, hidden, sorted,
-                     units, n_units, mu, y, stream);
-  if (rc) return rc;
+  if (xp == 1 && aligned16(x) && aligned16(gate_up) && aligned16(down) &&
+      gemm_shapes_ok(hidden, inter_dim, local_experts) &&
+      wide_units(tokens, hidden, inter_dim, local_experts, a)) {
+    const hipStream_t hs = (hipStream_t)stream;
+    if (!a_expert || !a_weight || !gate_up_scale || !down_scale || !dtype_index_ok(expert_dtype) ||
+        !dtype_float_ok(weight_dtype))
+      return MTPK_EINVAL;
+    const int64_t mw = local_experts + a / kWideTokens;  // no more than mu: a >= local_experts
+    const UnitSrc src = unit_list(units, sorted, n_units, mw);
+    const int64_t plane = a * inter_dim;
+    hipLaunchKernelGGL(k_moe_prep_wide, dim3(1), dim3(kPrepThreads), 0, hs, a_expert, expert_dtype,
+                       a_weight, weight_dtype, (int)a, expert_lo, (int)local_experts, sorted, units,
+                       (int)mw, n_units);
+    rc = launch_wide<true>(xplanes, tokens * hidden, 0, (int)hidden, gate_up, gate_up_scale,
+                           (int)inter_dim, src, top_k, inter, plane, nullptr, hs);
+    if (rc) return rc;
+    rc = launch_wide<false>(inter, 2 * plane, plane, (int)inter_dim, down, down_scale, (int)hidden, src,
+                            top_k, nullptr, 0, y, hs);
+    if (rc) return rc;
+  } else {
+    rc = mtpk_moe_prep(a_expert, expert_dtype, a_weight, weight_dtype, a, expert_lo, expert_hi,
+                       sorted, units, mu, n_units, stream);
+    if (rc) return rc;
+    rc = mtpk_moe_gate_up(xplanes, xp, tokens, hidden, gate_up, gate_up_scale, local_experts,
+                          inter_dim, sorted, units, n_units, mu, top_k, inter, ip, a, stream);
+    if (rc) return rc;
+    rc = mtpk_moe_down(inter, ip, a, inter_dim, down, down_scale, local_experts, hidden, sorted,
+                       units, n_units, mu, y, stream);
+    if (rc) return rc;
+  }
   const dim3 grid((unsigned)((hidden / 4 + 255) / 256), (unsigned)tokens);
   hipLaunchKernelGGL(tokens < kCombineWideTokens ? k_moe_combine<kCombineGroup> : k_moe_combine<4>,
                      grid, dim3(256), 0, (hipStream_t)stream, y, a_expert,
