@@ -37,7 +37,7 @@ constexpr int kPrepThreads = 1024;
 template <int NT>
 struct PrepSmem {
   static constexpr int kTot = MTPK_MAX_EXPERTS * 4;
-  static constexpr int kBytes = kTot + 2 * (NT / kWave) * 4;
+  static constexpr int kBytes = kTot + 3 * (NT / kWave) * 4;
 };
 
 // The counting sort on one workgroup of NT threads. The live test of a thread's first
@@ -45,16 +45,19 @@ struct PrepSmem {
 // then reloads the routing only past them.
 constexpr int kPrepKeep = 4;
 
-template <int NT, int kUnitTokens = mtpk::kUnitTokens, int kPrepKeep = mtpk::kPrepKeep>
+// WIDE > 0: from `min_live` live assignments on the units hold up to WIDE tokens and n_units[1] counts
+// them, else up to kUnitTokens and n_units[0]; the other count is 0.
+template <int NT, int kPrepKeep = mtpk::kPrepKeep, int WIDE = 0>
 __device__ inline void prep_body(const void* __restrict__ a_expert, int edt,
                                  const void* __restrict__ a_weight, int wdt, int assignments,
                                  int lo, int n_experts, int32_t* __restrict__ sorted,
                                  int32_t* __restrict__ units, int max_units,
-                                 int32_t* __restrict__ n_units, uint8_t* smem) {
+                                 int32_t* __restrict__ n_units, uint8_t* smem, int64_t min_live = 0) {
   constexpr int kPrepThreads = NT;
   int* cnt = reinterpret_cast<int*>(smem);
   int* wtot_c = reinterpret_cast<int*>(smem + PrepSmem<NT>::kTot);
   int* wtot_u = wtot_c + NT / kWave;
+  int* wtot_w = wtot_u + NT / kWave;
   const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
 
   int keep[kPrepKeep];  // local expert of assignment tid + i * NT, or -1 when it is dead
@@ -82,19 +85,22 @@ __device__ inline void prep_body(const void* __restrict__ a_expert, int edt,
   // (assignment count, unit count) pairs gives every expert its first position and first unit.
   const int per = (n_experts + kPrepThreads - 1) / kPrepThreads;
   const int e0 = tid * per;
-  int sc = 0, su = 0;
+  int sc = 0, su = 0, sw = 0;
   for (int i = 0; i < per; ++i) {
     const int e = e0 + i;
     if (e < n_experts) {
       const int c = cnt[e];
       sc += c;
       su += (c + kUnitTokens - 1) / kUnitTokens;
+      if (WIDE) sw += (c + WIDE - 1) / (WIDE ? WIDE : 1);
     }
   }
   const int ic = wave_incl_scan(sc, lane), iu = wave_incl_scan(su, lane);
+  const int iw = WIDE ? wave_incl_scan(sw, lane) : 0;
   if (lane == kWave - 1) {
     wtot_c[wv] = ic;
     wtot_u[wv] = iu;
+    if (WIDE) wtot_w[wv] = iw;
   }
   __syncthreads();
   int pc = ic - sc, pu = iu - su, total_units = 0;
@@ -105,24 +111,43 @@ __device__ inline void prep_body(const void* __restrict__ a_expert, int edt,
     }
     total_units += wtot_u[w];
   }
+  int ut = kUnitTokens;
+  bool wide = false;  // uniform
+  if (WIDE) {
+    int live = 0, units_w = 0, before = iw - sw;
+    for (int w = 0; w < kPrepThreads / kWave; ++w) {
+      live += wtot_c[w];
+      units_w += wtot_w[w];
+      if (w < wv) before += wtot_w[w];
+    }
+    wide = live >= min_live;
+    if (wide) {
+      ut = WIDE;
+      pu = before;
+      total_units = units_w;
+    }
+  }
   for (int i = 0; i < per; ++i) {
     const int e = e0 + i;
     if (e >= n_experts) break;
     const int c = cnt[e];
-    const int nu = (c + kUnitTokens - 1) / kUnitTokens;
+    const int nu = (c + ut - 1) / ut;
     for (int j = 0; j < nu; ++j) {
       const int u = pu + j;
       if (u < max_units) {
         units[3 * u + 0] = e;
-        units[3 * u + 1] = pc + j * kUnitTokens;
-        units[3 * u + 2] = min(kUnitTokens, c - j * kUnitTokens);
+        units[3 * u + 1] = pc + j * ut;
+        units[3 * u + 2] = min(ut, c - j * ut);
       }
     }
     cnt[e] = pc;  // from here on: the claim cursor of expert e
     pc += c;
     pu += nu;
   }
-  if (tid == 0) *n_units = min(total_units, max_units);
+  if (tid == 0) {
+    n_units[0] = wide ? 0 : min(total_units, max_units);
+    if (WIDE) n_units[1] = wide ? min(total_units, max_units) : 0;
+  }
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < kPrepKeep; ++i)
@@ -1408,11 +1433,11 @@ constexpr int kPrepWideKeep = 24;
 __global__ __launch_bounds__(kPrepThreads) void k_moe_prep_wide(
     const void* __restrict__ a_expert, int edt, const void* __restrict__ a_weight, int wdt,
     int assignments, int lo, int n_experts, int32_t* __restrict__ sorted,
-    int32_t* __restrict__ units, int max_units, int32_t* __restrict__ n_units) {
+    int32_t* __restrict__ units, int max_units, int32_t* __restrict__ n_units, int64_t min_live) {
   __shared__ __attribute__((aligned(16))) uint8_t smem[PrepSmem<kPrepThreads>::kBytes];
-  prep_body<kPrepThreads, kWideTokens, kPrepWideKeep>(a_expert, edt, a_weight, wdt, assignments, lo,
+  prep_body<kPrepThreads, kPrepWideKeep, kWideTokens>(a_expert, edt, a_weight, wdt, assignments, lo,
                                                       n_experts, sorted, units, max_units, n_units,
-                                                      smem);
+                                                      smem, min_live);
 }
 
 // ---------------------------------------------------------------- combine (unit mode)
@@ -1997,7 +2022,9 @@ UnitSrc unit_direct(const void* a_expert, int edt, const void* a_weight, int wdt
 // units hold a tile of 16 tokens either way, and the 16-token kernels, with their stores held back
 // and items pipelined, stream weights faster. 512 experts, top-10, Zipf(1.1), 16-token units against
 // wide ones: 256 rows (5 per expert) 539 / 579 us, 400 (8) 660 / 677, 600 (12) 803 / 797, 1024 (20)
-// 1047 / 929, 2048 (40) 1604 / 1259.
+// 1047 / 929, 2048 (40) 1604 / 1259. How many assignments are live is known only to the prep (a shard
+// of the experts sees every token's): the host takes these launches when there can be enough, the
+// prep chooses, and the other form's two launches find no unit (a few us).
 constexpr int64_t kWideMinPerExpert = 14;
 bool wide_units(int64_t tokens, int64_t hidden, int64_t inter_dim, int64_t local_experts, int64_t a) {
   constexpr int64_t lim = int64_t(1) << 31;
@@ -2321,16 +2348,22 @@ int mtpk_fused_moe_shared(const void* x, int x_dtype, int64_t tokens, int64_t hi
         !dtype_float_ok(weight_dtype))
       return MTPK_EINVAL;
     const int64_t mw = local_experts + a / kWideTokens;  // no more than mu: a >= local_experts
-    const UnitSrc src = unit_list(units, sorted, n_units, mw);
+    const UnitSrc src = unit_list(units, sorted, n_units + 1, mw);
+    const UnitSrc few = unit_list(units, sorted, n_units, mu);
     const int64_t plane = a * inter_dim;
     hipLaunchKernelGGL(k_moe_prep_wide, dim3(1), dim3(kPrepThreads), 0, hs, a_expert, expert_dtype,
                        a_weight, weight_dtype, (int)a, expert_lo, (int)local_experts, sorted, units,
-                       (int)mw, n_units);
+                       (int)mu, n_units, kWideMinPerExpert * local_experts);
     rc = launch_wide<true>(xplanes, tokens * hidden, 0, (int)hidden, gate_up, gate_up_scale,
                            (int)inter_dim, src, top_k, inter, plane, nullptr, hs);
     if (rc) return rc;
+    rc = launch_gate_up(1, xplanes, tokens * hidden, (int)hidden, gate_up, gate_up_scale, (int)inter_dim,
+                        few, mu, top_k, inter, plane, hs);
+    if (rc) return rc;
     rc = launch_wide<false>(inter, 2 * plane, plane, (int)inter_dim, down, down_scale, (int)hidden, src,
                             top_k, nullptr, 0, y, hs);
+    if (rc) return rc;
+    rc = launch_down_lds(inter, plane, (int)inter_dim, down, down_scale, (int)hidden, few, mu, y, hs);
     if (rc) return rc;
   } else {
     rc = mtpk_moe_prep(a_expert, expert_dtype, a_weight, weight_dtype, a, expert_lo, expert_hi,
