@@ -95,9 +95,13 @@ struct AttnIO {
   AttnRows gr;
 };
 
+// The gated output value. The sigmoid is exp2 and a reciprocal (1 ulp each; scaled, as the reciprocal of
+// a value above 2^126 would be flushed): for each of the 65536 gates the same bf16 value as with
+// expf and a division, which took a third of the prompt form's epilogue.
 __device__ inline uint16_t attn_gated(bool gated, uint16_t gate, float v) {
   if (!gated) return f32_to_bf16(v);
-  const float sg = bf16_to_f32(f32_to_bf16(1.f / (1.f + expf(-bf16_to_f32(gate)))));
+  const float e = __builtin_amdgcn_exp2f(-1.4426950408889634f * bf16_to_f32(gate));
+  const float sg = bf16_to_f32(f32_to_bf16(__builtin_amdgcn_rcpf((1.f + e) * 0x1p-32f) * 0x1p-32f));
   return f32_to_bf16(bf16_to_f32(f32_to_bf16(v)) * sg);
 }
 
@@ -386,8 +390,10 @@ int attention_slots(int hd, bool prompt) {
 
 // Rows per kv head from which a call takes the prompt form, one whole workgroup's: below, part of it
 // would be empty, and verify rounds (64 to 80 rows) read long contexts that the decode form streams.
-// 125 rows of 32 heads of 128: 18.7 against 19.5 us; 100 rows of 256 over 1500 cached keys: 33
-// against 40 us; 2047 rows: 98 against 392 us.
+// From there on it is the faster one over every lane count and context: against the decode form, at
+// exactly 128 rows, one lane of 256 over 128 keys 23 / 37 us and over 8192 28 / 48, 48 lanes over 600
+// keys 36 / 47, over 2000 66 / 101 and over 8192 185 / 352; 48 lanes of 128 over 8192 keys 181 / 335;
+// 2047 rows over themselves 115 / 382.
 constexpr int64_t kPromptMinRows = 128;
 bool attention_prompt(int64_t rows) { return rows >= kPromptMinRows; }
 int64_t attention_row_groups(int64_t rows);

@@ -10,17 +10,19 @@
 // Row m of a K tile is its key with bits 2 and 3 of m swapped: then the S^T values that a lane gets
 // (query row l % 32, rows 8 i + 4 (l / 32) + 0..3 of the tile) are 8 adjacent keys of each 16, which
 // is the B operand of O^T with V^T read 16 bytes at a time, so P never leaves its registers. The
-// row maximum needs one exchange with lane l ^ 32, and the rescaling of O is a lane's own factor;
-// the reference exponent m only moves when a score lies more than 2^8 above it (P then stays
-// below 2^8, with the same relative error), so most tiles skip the rescaling. Tiles of 32 keys go
-// straight to LDS, one tile ahead, in two buffers with one barrier per tile; their 16-byte pieces
-// are permuted on the way (by the key, or by the channel) so that the reads fall on all banks.
+// row maximum needs one exchange with lane l ^ 32, and the rescaling of O is a lane's own factor.
+// The reference exponent of a row moves with its maximum, as in the decode form, so that the largest
+// P is exactly 1: error against 64 bits at 2047 rows 3.07e-3 in both forms, and nearly all outputs
+// the same bits (moved only once a score lay 2^8 above it, P of the largest key was a rounded
+// value: 3.13e-3, at 103 us). Tiles of 32 keys go straight to LDS, one tile ahead, in two
+// buffers with one barrier per tile; their 16-byte pieces are permuted on the way (by the key, or by
+// the channel) so that the reads fall on all banks.
 //
-// 98 us at 2047 rows of 32 heads of 256 on 2 kv heads (69 GFLOP: 0.70 PFLOP/s) against 392 us for
+// 115 us at 2047 rows of 32 heads of 256 on 2 kv heads (69 GFLOP: 0.60 PFLOP/s) against 382 us for
 // the decode form, which runs every row group over all keys with 16 rows a wave. What is
-// left: the heaviest workgroup's 64 tiles one after another (products, softmax, products), whose
-// CU partner ends early. Two teams of four waves on alternate tiles in one workgroup halved that
-// chain but run in lockstep, matrix unit and softmax taking turns: 126 us.
+// left: the heaviest workgroup's 64 tiles one after another (products, softmax, rescaling, products),
+// whose CU partner ends early. Two teams of four waves on alternate tiles in one workgroup halved
+// that chain but run in lockstep, matrix unit and softmax taking turns: slower by a quarter.
 #pragma once
 
 #include "mtpk_device.h"
@@ -52,14 +54,6 @@ __device__ inline int prompt_swap(int i) { return (i & ~12) | ((i & 4) << 1) | (
 // The change of place of a K row's pieces: the rows 0..3 and 0..7 that one LDS cycle reads, of either
 // half of the wave, then lie in different bank groups.
 __device__ inline int prompt_flip(int row) { return ((row & 3) << 1) | (row >> 2 & 1); }
-
-// attn_gated's value for an output already rounded to bf16, with the sigmoid as exp2 and a reciprocal
-// (each 1 ulp, before the rounding of the sigmoid to bf16).
-__device__ inline uint16_t prompt_gated(uint16_t gate, uint16_t v) {
-  const float e = __builtin_amdgcn_exp2f(-1.4426950408889634f * bf16_to_f32(gate));
-  const float sg = bf16_to_f32(f32_to_bf16(__builtin_amdgcn_rcpf(1.f + e)));
-  return f32_to_bf16(bf16_to_f32(v) * sg);
-}
 
 template <int HD>
 __global__ __launch_bounds__(256, 2) void k_prompt_attention(
@@ -197,7 +191,7 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attention(
     for (int i = 1; i < 16; ++i) tm = fmaxf(tm, s[i]);
     tm = fmaxf(tm, __shfl_xor(tm, 32, kWave));
     const float mn = fmaxf(m, tm * scale_log2);
-    if (__ballot(mn > m + 8.f || (m == -INFINITY && mn > m)) != 0ull) {  // uniform over the wave
+    if (__ballot(mn > m) != 0ull) {  // uniform over the wave
       const float alpha = mn == -INFINITY ? 1.f : exp2f(m - mn);
       m = mn;
       l *= alpha;
@@ -211,7 +205,7 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attention(
     float part[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const float e = __builtin_amdgcn_exp2f(fmaf(s[i], scale_log2, -ms));  // in [0, 2^8]; 0 below 2^-126
+      const float e = __builtin_amdgcn_exp2f(fmaf(s[i], scale_log2, -ms));  // in [0, 1]; 0 below 2^-126
       part[i & 3] += e;
       p[i >> 3][i & 7] = (__bf16)e;
     }
@@ -264,8 +258,8 @@ __global__ __launch_bounds__(256, 2) void k_prompt_attention(
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          w[e] = (uint32_t)prompt_gated((uint16_t)(g[e] & 0xffffu), (uint16_t)(w[e] & 0xffffu)) |
-                 ((uint32_t)prompt_gated((uint16_t)(g[e] >> 16), (uint16_t)(w[e] >> 16)) << 16);
+          w[e] = (uint32_t)attn_gated(true, (uint16_t)(g[e] & 0xffffu), bits_f32(w[e] << 16)) |
+                 ((uint32_t)attn_gated(true, (uint16_t)(g[e] >> 16), bits_f32(w[e] & 0xffff0000u)) << 16);
       }
       if (wide) {  // uniform: output and gate rows on 16-byte boundaries
         *reinterpret_cast<u32x4_t*>(orow) = w;

@@ -73,3 +73,58 @@ def test_merge_of_many_splits(dev, t, base) -> None:
     got = attention.paged_attention(q.to(dev), k.to(dev), attention.v_blocks(v).to(dev), torch.from_numpy(table).to(dev),
                                     torch.from_numpy(pos).to(dev), max(base) + t, 0.09)
     _compare(got, want)
+
+
+def _tile_by_tile(q, keys, vals, gate, group, scale):
+    """The decode form's arithmetic on one lane without cached keys, one split: online softmax over
+    tiles of 32 keys whose reference is the row's running maximum, fp32 sums, bf16 probabilities."""
+    heads, t, hd = q.shape
+    k, v = (x.float().repeat_interleave(group, dim=1).transpose(0, 1).contiguous() for x in (keys, vals))
+    live = torch.arange(t, device=q.device)[None, :] <= torch.arange(t, device=q.device)[:, None]
+    s = (q.float() @ k.transpose(1, 2).contiguous() * scale * 1.4426950408889634).masked_fill(~live, -torch.inf)
+    m = torch.full((heads, t, 1), -torch.inf, device=q.device)
+    l, o = torch.zeros_like(m), torch.zeros(heads, t, hd, device=q.device)
+    for k0 in range(0, t, 32):
+        x = s[..., k0 : k0 + 32]
+        mn = torch.maximum(m, x.amax(-1, keepdim=True))
+        e, alpha = torch.exp2(x - mn), torch.exp2(m - mn)
+        l, m = l * alpha + e.sum(-1, keepdim=True), mn
+        o = o * alpha + e.bfloat16().float() @ v[:, k0 : k0 + 32]
+    out = (o / l).bfloat16()
+    return out * torch.sigmoid(gate) if gate is not None else out
+
+
+@pytest.mark.parametrize("heads,kvh,hd,t", [(32, 2, 256, 300), (16, 4, 128, 160), (8, 2, 64, 200)])
+def test_prompt_rows_round_as_the_decode_form(dev, heads, kvh, hd, t) -> None:
+    """Probabilities are rounded against the row's running maximum (the largest is exactly 1) and the
+    sigmoid is the decode form's, so only fp32 sums in another order (about 2^-20) differ: they move
+    about 2^-10 of the bf16 outputs to a neighbour. Rounding against a stale maximum moves a third."""
+    q, k, v, table, pos = _case(11, 1, heads, kvh, hd, t, [0], t // 16 + 2)
+    rows = torch.from_numpy(table[0].repeat(16) * 16 + np.tile(np.arange(16), table.shape[1]))[:t].long()
+    qd = q.to(dev)[0]
+    gate = torch.randn(1, t, heads, hd, device=dev).bfloat16()
+    args = (k.to(dev), attention.v_blocks(v).to(dev), torch.from_numpy(table).to(dev), torch.from_numpy(pos).to(dev),
+            t, hd**-0.5)
+    for g in (None, gate):
+        got = attention.paged_attention_gated(q.to(dev).transpose(1, 2).contiguous(), *args, g)[0].transpose(0, 1)
+        want = _tile_by_tile(qd, k[rows].to(dev), v[rows].to(dev), None if g is None else g[0].transpose(0, 1),
+                             heads // kvh, hd**-0.5)
+        assert float((got != want).float().mean()) < 4 * 2**-10
+
+
+@pytest.mark.parametrize("t,base", [(64, 0), (4, 2100)])
+def test_every_gate_value(dev, t, base) -> None:
+    """One visible value of 1 (all cached values are 1): the output is the sigmoid of the gate, for every
+    bf16 gate, in the prompt form's own epilogue and in the merge of the key splits."""
+    heads, kvh, hd = 16, 1, 64
+    q, k, v, table, pos = _case(12, 1, heads, kvh, hd, t, [base], (base + t) // 16 + 2)
+    args = (k.to(dev), attention.v_blocks(torch.ones_like(v)).to(dev), torch.from_numpy(table).to(dev),
+            torch.from_numpy(pos).to(dev), base + t, 0.01)
+    every = torch.arange(65536, device=dev).to(torch.int16).view(torch.bfloat16)
+    n = t * heads * hd
+    for i in range(0, 65536, n):
+        gate = every[i : i + n].view(1, t, heads, hd)
+        got = attention.paged_attention_gated(q.to(dev).transpose(1, 2).contiguous(), *args, gate)
+        want = torch.sigmoid(gate.float()).bfloat16()
+        assert torch.equal(got.isnan(), want.isnan())
+        assert torch.equal(got.nan_to_num(), want.nan_to_num())
