@@ -19,6 +19,8 @@
 // With n_split > 1 every workgroup writes its unnormalised O with (m, l) per row and a second
 // kernel merges the splits; with one split the workgroup writes the bf16 output directly.
 
+#include <algorithm>
+
 #include "mtpk_device.h"
 #include "mtpk_host.h"
 
@@ -410,10 +412,23 @@ int64_t attention_row_groups(int64_t rows) {
 // for its whole length, and every extra split adds partials to the merge: at 48 lanes, 2 kv
 // heads of 256 and 8192 keys (96 workgroups per split, 512 slots), 5 splits take 179 us per
 // call against 199 us for 8 and 10 and 220 us for 12 and 16.
+//
+// The prompt form at head_dim 256 keeps a CU's matrix unit busy with one workgroup, and its
+// partials are 1 KB a row: one workgroup per CU is enough unless that leaves a split more than
+// kPromptSplitTiles tiles one after another. 900 rows over themselves 59 us in one split, 68 in two;
+// 200 rows over 2000 cached keys 41 in 5, 46 in 8; 16 lanes of 8 rows over 8192 keys 71 in 8, 84
+// in 16; but 500 rows over 8000 keys 195 in 2, 172 in 4, 48 lanes of 9 rows over 2000 keys 100 in 1,
+// 79 in 2, and 48 lanes of 8 rows over 8192 keys 215 in 2, 188 in 5. Smaller heads gain from a
+// second and third workgroup (1300 rows of 128: 46 us in one split, 41 in 4).
+constexpr int64_t kPromptSplitTiles = 48;
 int attention_splits(int hd, int64_t B, int64_t kvh, int64_t rows, int64_t max_ctx) {
   const int64_t wgs = B * kvh * attention_row_groups(rows);
-  const int64_t fit = attention_slots(hd, attention_prompt(rows)) / (wgs > 0 ? wgs : 1);
+  int64_t fit = attention_slots(hd, attention_prompt(rows)) / (wgs > 0 ? wgs : 1);
   const int64_t tiles = (max_ctx + kAttnKeys - 1) / kAttnKeys;
+  if (hd == 256 && attention_prompt(rows)) {
+    const int64_t one = std::max<int64_t>(device_cu_count() / (wgs > 0 ? wgs : 1), 1);
+    if (tiles <= one * kPromptSplitTiles) fit = one;
+  }
   const int64_t cap = tiles / 8 > 1 ? tiles / 8 : 1;  // at least 8 tiles per split
   int64_t n = fit < cap ? fit : cap;
   if (n > kMergeSplits) n = kMergeSplits;
