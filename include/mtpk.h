@@ -456,8 +456,8 @@ int mtpk_delta_rule(float* state, int64_t slots_total, const int64_t* slot, int6
  * a (row, head) whose k is longer than 1, whose g is positive, whose beta lies outside [0, 1] or
  * whose v, k, g or beta is not finite runs step by step as before. The bytes cover one row or
  * more; rows run in groups that fit, so a larger workspace takes fewer launches. workspace is
- * 256-byte aligned. Where it is 0, or with operands that are not 16-byte aligned, the call is
- * mtpk_delta_rule (workspace unused, may be NULL). */
+ * 256-byte aligned. Where the bytes are 0 (always below 16 steps), or with operands that are not
+ * 16-byte aligned, the call is mtpk_delta_rule (workspace unused, may be NULL). */
 int64_t mtpk_delta_rule_workspace_bytes(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads,
                                         int64_t k_dim, int64_t v_dim, int want_out);
 int mtpk_delta_rule_ws(float* state, int64_t slots_total, const int64_t* slot, int64_t rows, int64_t t,

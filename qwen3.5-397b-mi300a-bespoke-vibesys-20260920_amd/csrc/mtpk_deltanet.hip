@@ -17,6 +17,8 @@
 // state is not written. Commit mode: row j replays its accepted prefix, min(lengths[j], t)
 // steps, and stores the advanced state over its slot (outputs optional).
 
+#include <algorithm>
+
 #include "mtpk_deltanet_chunk.h"
 #include "mtpk_device.h"
 #include "mtpk_host.h"
@@ -346,24 +348,34 @@ int64_t dn_chunk_row_bytes(int64_t t, int64_t heads, int64_t qk_heads, bool want
 }
 
 // Whether a call's sizes are for the chunk form: its shapes (32-bit byte offsets inside a row), and
-// the faster of the two by these fits, in us. m counts matrices of 64 heads of 128 x 128. Step by
-// step a step takes 2.1 us (1.5 read back to back) while every wave is resident and more as rows are
-// added; the chunks cost two launches and 64 steps' products, which fill the chip from m = 1 on.
-// Step by step / chunks, with outputs: m = 1, 24 steps 55 / 30, 1500 steps 2286 / 180; m = 4, 24
-// steps 67 / 67, 128 steps 319 / 120; m = 16, 48 steps 163 / 204, 128 steps 430 / 369; m = 48, 128
-// steps 1011 / 1121. Commits: m = 1, 24 steps 26 / 25, 1500 steps 1637 / 116; m = 4, 48 steps
-// 60 / 52; m = 16, 128 steps 183 / 238.
+// the faster of the two by these fits, in us. m counts matrices of 64 heads of 128 x 128. A step of
+// the step-by-step form is a dependent pass that hides behind the other waves only as rows are
+// added; a chunk's products fill the chip from m = 1 on and then grow with m, a little faster than
+// linearly as the operands outgrow the caches. Step by step / chunks, with outputs: m = 1, 16 steps
+// 24 / 29, 24 steps 35 / 29, 1500 steps 2286 / 178; m = 2, 24 steps 36 / 42, 40 steps 57 / 44; m = 4, 32
+// steps 57 / 68, 64 steps 107 / 69, 65 steps 108 / 113, 128 steps 207 / 116; m = 8, 64 steps 107 / 118,
+// 129 steps 209 / 248, 256 steps 400 / 314; m = 16, 320 steps 643 / 785. Commits: m = 1, 24 steps
+// 26 / 25, 1500 steps 1637 / 116; m = 4, 64 steps 76 / 51, 65 steps 77 / 74; m = 8, 64 steps 81 / 87, 128
+// steps 149 / 131. Near the line the old form keeps the call (the factor 1.05).
+constexpr int64_t kDnChunkMinSteps = 16;  // no call of fewer steps takes the chunk form
 bool dn_chunk_fits(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads, int64_t k_dim, int64_t v_dim,
                    bool want_out) {
-  if (k_dim != kDnChunkDk || v_dim % (4 * kWave / kDnKG) != 0 ||
+  if (t < kDnChunkMinSteps || k_dim != kDnChunkDk || v_dim % (4 * kWave / kDnKG) != 0 ||
       (t + kDnChunk) * (qk_heads * k_dim > heads * v_dim ? qk_heads * k_dim : heads * v_dim) * 4 >=
           (int64_t(1) << 31))
     return false;
   const double m = (double)rows * heads * v_dim / (64 * 128), n = (double)((t + kDnChunk - 1) / kDnChunk);
-  const double least = want_out ? 6.0 : 3.6, full = m * (want_out ? 10.3 : 6.2);
-  const double chunks = 20.0 + n * (full > least ? full : least);
-  const double steps = t * (want_out ? 2.1 + 0.075 * m : 0.95 + 0.03 * m);
-  return chunks < steps;
+  double launch, chunk, steps;
+  if (want_out) {
+    launch = std::max(20.0, 14 + 10 * std::min(m, 5.0));
+    chunk = std::max(5.5, 6.2 * m + 0.18 * m * m);
+    steps = 1.5 + 0.75 * m + t * (1.38 + 0.03 * m);
+  } else {
+    launch = std::max(19.0, 15 + 5.5 * std::min(m, 7.0));
+    chunk = std::max(3.6, 3.9 * m + 0.07 * m * m);
+    steps = 3 + 1.2 * m + t * (0.9 + 0.02 * m);
+  }
+  return 1.05 * (launch + n * chunk) < steps;
 }
 
 DnChunkWs dn_chunk_ws(void* workspace, int64_t rows, int64_t t, int64_t heads, int64_t qk_heads,

@@ -22,6 +22,8 @@ import _mtpk
 def _steps_workspace(rows: int, t: int, heads: int, qk_heads: int, k_dim: int, v_dim: int, want_out: bool,
                      device: torch.device) -> torch.Tensor | None:
     """Scratch of a call of many steps (`mtpk_delta_rule_workspace_bytes`), None where it takes none."""
+    if t < 16:  # never any: a decode or verify round's call asks for nothing
+        return None
     n = int(_mtpk.lib().mtpk_delta_rule_workspace_bytes(rows, t, heads, qk_heads, k_dim, v_dim, int(want_out)))
     return torch.empty(n, dtype=torch.uint8, device=device) if n > 0 else None
 
