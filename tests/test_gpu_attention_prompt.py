@@ -32,6 +32,8 @@ def _compare(got, want):
     (6, 2, 128, 50, [3]),         # a group that does not divide a row group
     (32, 2, 256, 12, [2100, 40]),  # many splits, one lane's mostly empty
     (4, 4, 64, 200, [0]),         # no grouping
+    (32, 2, 256, 1100, [0]),      # 276 workgroups: more than CUs, all resident (the paired order)
+    (32, 2, 256, 300, [1300]),    # 256 wide, many row groups in several splits
 ])
 def test_prompt_rows_match_the_oracle(dev, heads, kvh, hd, t, base) -> None:
     blocks = (max(base) + t + 15) // 16 + 1
