@@ -164,7 +164,7 @@ __device__ __forceinline__ void delta_rule_kg_body(
     int bid, float* __restrict__ state, int64_t slots_total, const int64_t* __restrict__ slot, int t,
     int heads, int rep, int dv, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ g, const float* __restrict__ beta,
-    const int64_t* __restrict__ lengths, float* __restrict__ out) {
+    const int64_t* __restrict__ lengths, float* __restrict__ out, DnPiece piece = {0, nullptr}) {
   static_assert(KG == 4 || KG == 8, "row groups of 32 or 16");
   constexpr int DK = 128, QR = DK / KG, CW = 4 * kWave / KG;  // rows per group, columns per wave
   const int nblk = dv / CW;
@@ -180,13 +180,15 @@ __device__ __forceinline__ void delta_rule_kg_body(
       for (int st = 0; st < t; ++st) out[((int64_t)row * t + st) * heads * dv + o_row] = 0.f;
     return;  // uniform over the one-wave workgroup
   }
-  const rsrc_t rsm = make_rsrc(state + ((s_idx * heads + head) * DK) * (int64_t)dv, (uint32_t)(DK * dv * 4));
+  float* const pool = state + ((s_idx * heads + head) * DK) * (int64_t)dv;
+  float* const kept = piece.carry ? piece.carry + (int64_t)head * DK * dv : pool;  // one row
+  const rsrc_t rsm = make_rsrc(kept, (uint32_t)(DK * dv * 4));
+  const rsrc_t rsi = make_rsrc(piece.t0 > 0 ? kept : pool, (uint32_t)(DK * dv * 4));
   const uint32_t voff = ((uint32_t)(QR * kg) * (uint32_t)dv + (uint32_t)col4) * 4u, drow = (uint32_t)dv * 4u;
   f32x4_t s[QR];  // s[i] = row QR kg + i, columns col4 .. col4 + 3
 #pragma unroll
-  for (int i = 0; i < QR; ++i) s[i] = __builtin_bit_cast(f32x4_t, buf16(rsm, voff, drow * (uint32_t)i));
-  int n = t;
-  if (COMMIT) n = (int)min(max(lengths[row], (int64_t)0), (int64_t)t);
+  for (int i = 0; i < QR; ++i) s[i] = __builtin_bit_cast(f32x4_t, buf16(rsi, voff, drow * (uint32_t)i));
+  const int n = COMMIT ? dn_steps(lengths, row, t, piece.t0) : t;
   const int qk_heads = heads / rep, kh = head / rep;
   // k and q pass through LDS as in the general form; step st + 1's inputs load while step st runs
   __shared__ __attribute__((aligned(16))) float kq[2][2][DK];
@@ -331,20 +333,43 @@ __global__ __launch_bounds__(kWave, (OUT && COMMIT) ? 2 : 3) void k_delta_rule_r
     int heads, int rep, int dv, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ g, const float* __restrict__ beta,
     const int64_t* __restrict__ lengths, float* __restrict__ out, const int32_t* __restrict__ odd,
-    int nch) {
+    int nch, DnPiece piece) {
   const int bh = (int)blockIdx.x / (dv / (4 * kWave / kDnKG));
-  if (!dn_left_over(odd, nch, bh, lengths, bh / heads, t)) return;  // uniform
+  if (!dn_left_over(odd, nch, bh, lengths, bh / heads, t, piece.t0)) return;  // uniform
   delta_rule_kg_body<kDnKG, OUT, COMMIT>((int)blockIdx.x, state, slots_total, slot, t, heads, rep, dv,
-                                         q, k, v, g, beta, lengths, out);
+                                         q, k, v, g, beta, lengths, out, piece);
 }
 
+// The scratch of a call: rows run in groups that fit, and a row that does not fit in pieces of whole
+// chunks, one after another, which gives the same bits. 57 KB a step of 64 heads with outputs: a row
+// of up to 4600 steps is one piece.
 constexpr int64_t kDnChunkWsBytes = int64_t(256) << 20;
 
-// Workspace of one row of a chunked call (a multiple of 256 bytes).
-int64_t dn_chunk_row_bytes(int64_t t, int64_t heads, int64_t qk_heads, bool want_out) {
-  const int64_t nch = (t + kDnChunk - 1) / kDnChunk, m = want_out ? 2 : 1;
+// Workspace of one row's `nch` chunks (a multiple of 256 bytes).
+int64_t dn_chunk_row_bytes(int64_t nch, int64_t heads, int64_t qk_heads, bool want_out) {
+  const int64_t m = want_out ? 2 : 1;
   return qk_heads * nch * (m + 1) * kDnRowTiles * kDnTile * 4 +
          heads * nch * (m * kDnSqTiles * kDnTile + 2 * kDnChunk) * 4 + align256(heads * nch * 4);
+}
+
+// How a call's rows and chunks go into `bytes` of workspace: `rows` rows of `nch` chunks at once, or one
+// row in pieces of `nch` chunks (then with the carried state of a call with outputs behind
+// them). nch = 0: not even one chunk fits.
+struct DnPlan {
+  int64_t rows, nch, bytes;
+  bool pieces;
+};
+DnPlan dn_chunk_plan(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads, int64_t v_dim, bool want_out,
+                     int64_t bytes) {
+  const int64_t nch = (t + kDnChunk - 1) / kDnChunk, one = dn_chunk_row_bytes(nch, heads, qk_heads, want_out);
+  if (one <= bytes) {
+    const int64_t fit = std::min(bytes / one, rows);
+    return {fit, nch, fit * one, false};
+  }
+  const int64_t carry = want_out ? align256(heads * kDnChunkDk * v_dim * 4) : 0;
+  const int64_t per = dn_chunk_row_bytes(1, heads, qk_heads, want_out);  // no less than one chunk's share
+  const int64_t fit = bytes > carry ? (bytes - carry) / per : 0;
+  return {1, fit, dn_chunk_row_bytes(fit, heads, qk_heads, want_out) + carry, true};
 }
 
 // Whether a call's sizes are for the chunk form: its shapes (32-bit byte offsets inside a row), and
@@ -378,9 +403,8 @@ bool dn_chunk_fits(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads, int
   return 1.05 * (launch + n * chunk) < steps;
 }
 
-DnChunkWs dn_chunk_ws(void* workspace, int64_t rows, int64_t t, int64_t heads, int64_t qk_heads,
+DnChunkWs dn_chunk_ws(void* workspace, int64_t rows, int64_t nch, int64_t heads, int64_t qk_heads,
                       bool want_out) {
-  const int64_t nch = (t + kDnChunk - 1) / kDnChunk;
   const int64_t kq = rows * qk_heads * nch * kDnRowTiles * kDnTile, slabs = rows * heads * nch;
   const int64_t sq = slabs * kDnSqTiles * kDnTile;
   DnChunkWs w{};
@@ -403,21 +427,27 @@ DnChunkWs dn_chunk_ws(void* workspace, int64_t rows, int64_t t, int64_t heads, i
   return w;
 }
 
-// The chunk launches of `rows` rows: prep and scan. The caller launches what the scan left.
+// The launches of `rows` rows: prep, scan, and what the scan left.
 template <bool OUT, bool COMMIT>
-int launch_dn_chunks(float* state, int64_t slots_total, const int64_t* slot, int rows, int t, int heads,
-                     int qk_heads, int dv, const float* q, const float* k, const float* v,
+int launch_dn_chunks(float* state, int64_t slots_total, const int64_t* slot, int64_t rows, int64_t t, int64_t heads,
+                     int64_t qk_heads, int64_t dv, const float* q, const float* k, const float* v,
                      const float* g, const float* beta, const int64_t* lengths, float* out,
-                     const DnChunkWs& ws, hipStream_t st) {
-  const int nch = (t + kDnChunk - 1) / kDnChunk;
-  const int64_t pg = (int64_t)rows * qk_heads * nch, sg = (int64_t)rows * heads * (dv / kDnScanCols);
+                     const DnChunkWs& ws, DnPiece piece, hipStream_t st) {
+  const int64_t nch = (t + kDnChunk - 1) / kDnChunk;
+  const int64_t pg = rows * qk_heads * nch, sg = rows * heads * (dv / kDnScanCols);
   if (pg > INT32_MAX || sg > INT32_MAX) return MTPK_EINVAL;
-  hipLaunchKernelGGL((k_dn_chunk_prep<OUT>), dim3((unsigned)pg), dim3(256), 0, st, t, heads, qk_heads, dv, nch, q,
-                     k, v, g, beta, lengths, ws);
-  const int rc = status_of(hipGetLastError());
+  hipLaunchKernelGGL((k_dn_chunk_prep<OUT>), dim3((unsigned)pg), dim3(256), 0, st, (int)t, (int)heads,
+                     (int)qk_heads, (int)dv, (int)nch, q, k, v, g, beta, lengths, ws, piece.t0);
+  int rc = status_of(hipGetLastError());
   if (rc) return rc;
-  hipLaunchKernelGGL((k_dn_chunk_scan<OUT, COMMIT>), dim3((unsigned)sg), dim3(256 * kDnScanTiles), 0, st, state, slots_total,
-                     slot, t, heads, qk_heads, dv, nch, v, lengths, out, ws, rows * heads);
+  hipLaunchKernelGGL((k_dn_chunk_scan<OUT, COMMIT>), dim3((unsigned)sg), dim3(256 * kDnScanTiles), 0, st, state,
+                     slots_total, slot, (int)t, (int)heads, (int)qk_heads, (int)dv, (int)nch, v, lengths, out, ws,
+                     (int)(rows * heads), piece);
+  rc = status_of(hipGetLastError());
+  if (rc) return rc;
+  hipLaunchKernelGGL((k_delta_rule_rest<OUT, COMMIT>), dim3((unsigned)(rows * heads * (dv / (4 * kWave / kDnKG)))),
+                     dim3(kWave), 0, st, state, slots_total, slot, (int)t, (int)heads, (int)(heads / qk_heads),
+                     (int)dv, q, k, v, g, beta, lengths, out, ws.odd, (int)nch, piece);
   return status_of(hipGetLastError());
 }
 
@@ -804,9 +834,8 @@ int64_t mtpk_delta_rule_workspace_bytes(int64_t rows, int64_t t, int64_t heads, 
       v_dim <= 0 || v_dim > 4096)
     return 0;
   if (!dn_chunk_fits(rows, t, heads, qk_heads, k_dim, v_dim, want_out != 0)) return 0;
-  const int64_t one = dn_chunk_row_bytes(t, heads, qk_heads, want_out != 0);
-  const int64_t fit = kDnChunkWsBytes / one;
-  return one * (fit < 1 ? 1 : fit < rows ? fit : rows);
+  const DnPlan plan = dn_chunk_plan(rows, t, heads, qk_heads, v_dim, want_out != 0, kDnChunkWsBytes);
+  return plan.nch > 0 ? plan.bytes : 0;
 }
 
 int mtpk_delta_rule_ws(float* state, int64_t slots_total, const int64_t* slot, int64_t rows, int64_t t,
@@ -821,39 +850,34 @@ int mtpk_delta_rule_ws(float* state, int64_t slots_total, const int64_t* slot, i
       mtpk_delta_rule_workspace_bytes(rows, t, heads, qk_heads, k_dim, v_dim, out != nullptr) <= 0)
     return mtpk_delta_rule(state, slots_total, slot, rows, t, heads, qk_heads, k_dim, v_dim, q, k, v, g,
                            beta, lengths, out, stream);
-  const int64_t one = dn_chunk_row_bytes(t, heads, qk_heads, out != nullptr), fit = workspace_bytes / one;
-  if (fit < 1) return MTPK_EINVAL;
+  const bool want_out = out != nullptr;
+  const DnPlan least = dn_chunk_plan(1, t, heads, qk_heads, v_dim, want_out, kDnChunkWsBytes);
+  if (workspace_bytes < least.bytes) return MTPK_EINVAL;
+  const DnPlan plan = dn_chunk_plan(rows, t, heads, qk_heads, v_dim, want_out, workspace_bytes);
   const hipStream_t st = (hipStream_t)stream;
-  const int rep = (int)(heads / qk_heads), nch = (int)((t + kDnChunk - 1) / kDnChunk);
-  for (int64_t r0 = 0; r0 < rows; r0 += fit) {  // as many rows at once as the workspace holds
-    const int r = (int)(rows - r0 < fit ? rows - r0 : fit);
-    const DnChunkWs ws = dn_chunk_ws(workspace, r, t, heads, qk_heads, out != nullptr);
-    const int64_t qo = r0 * t * qk_heads * k_dim, vo = r0 * t * heads * v_dim, go = r0 * t * heads;
+  for (int64_t r0 = 0; r0 < rows; r0 += plan.rows) {  // as many rows at once as the workspace holds
+    const int64_t r = std::min(plan.rows, rows - r0);
+    const DnChunkWs ws = dn_chunk_ws(workspace, r, plan.nch, heads, qk_heads, want_out);
+    // the carried state lies at the workspace's end
+    float* const carry = plan.pieces && !lengths
+        ? reinterpret_cast<float*>(static_cast<char*>(workspace) + dn_chunk_row_bytes(plan.nch, heads, qk_heads, want_out))
+        : nullptr;
     const int64_t* const ln = lengths ? lengths + r0 : nullptr;
-    float* const o = out ? out + vo : nullptr;
     float* const stt = slot ? state : state + r0 * heads * k_dim * v_dim;  // no slots: row j is slot j
     const int64_t* const sl = slot ? slot + r0 : nullptr;
     const int64_t total = slot ? slots_total : slots_total - r0;
-    int rc;
-    const unsigned grid = (unsigned)(r * heads * (v_dim / (4 * kWave / kDnKG)));
-#define MTPK_DNC(OUT_, COMMIT_)                                                                      \
-  rc = launch_dn_chunks<OUT_, COMMIT_>(stt, total, sl, r, (int)t, (int)heads,                       \
-                                       (int)qk_heads, (int)v_dim, q + qo, k + qo, v + vo, g + go,    \
-                                       beta + go, ln, o, ws, st);                                    \
-  if (rc) return rc;                                                                                 \
-  hipLaunchKernelGGL((k_delta_rule_rest<OUT_, COMMIT_>), dim3(grid), dim3(kWave), 0, st, stt,        \
-                     total, sl, (int)t, (int)heads, rep, (int)v_dim, q + qo, k + qo,    \
-                     v + vo, g + go, beta + go, ln, o, ws.odd, nch);
-    if (!lengths) {
-      MTPK_DNC(true, false)
-    } else if (out) {
-      MTPK_DNC(true, true)
-    } else {
-      MTPK_DNC(false, true)
-    }
+    for (int64_t t0 = 0; t0 < t; t0 += plan.nch * kDnChunk) {  // one pass unless a row goes in pieces
+      const int64_t n = std::min(t - t0, plan.nch * kDnChunk), s0 = r0 * t + t0;
+      const int64_t qo = s0 * qk_heads * k_dim, vo = s0 * heads * v_dim, go = s0 * heads;
+      float* const o = out ? out + vo : nullptr;
+      const DnPiece piece{(int)t0, carry};
+#define MTPK_DNC(OUT_, COMMIT_)                                                                               \
+  launch_dn_chunks<OUT_, COMMIT_>(stt, total, sl, r, n, heads, qk_heads, v_dim, q + qo, k + qo, v + vo, g + go, \
+                                  beta + go, ln, o, ws, piece, st)
+      const int rc = !out ? MTPK_DNC(false, true) : lengths || carry ? MTPK_DNC(true, true) : MTPK_DNC(true, false);
 #undef MTPK_DNC
-    rc = status_of(hipGetLastError());
-    if (rc) return rc;
+      if (rc) return rc;
+    }
   }
   return 0;
 }

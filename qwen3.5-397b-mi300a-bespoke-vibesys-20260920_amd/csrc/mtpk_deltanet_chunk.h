@@ -57,9 +57,17 @@ struct DnChunkWs {
 constexpr int kDnTile = 256;                  // floats of a tile
 constexpr int kDnRowTiles = 32, kDnSqTiles = 16;  // tiles of a [64][128] and of a [64][64] matrix
 
-// Steps row `row` runs and its slot, or n = 0 when there is nothing to do.
-__device__ inline int dn_steps(const int64_t* lengths, int row, int t) {
-  return lengths ? (int)min(max(lengths[row], (int64_t)0), (int64_t)t) : t;
+// A piece of a call's steps whose scratch would pass the workspace: its first step (`lengths` count
+// from the call's first), and in verify calls, whose pool keeps its values, a [heads][k_dim][v_dim]
+// matrix set that carries the one row's state from piece to piece. A whole call has {0, null}.
+struct DnPiece {
+  int t0;
+  float* carry;
+};
+
+// Steps of the piece that row `row` runs.
+__device__ inline int dn_steps(const int64_t* lengths, int row, int t, int t0) {
+  return lengths ? (int)min(max(lengths[row] - t0, (int64_t)0), (int64_t)t) : t;
 }
 
 // e^x of an fp64 exponent, to fp32 accuracy: rounding x to fp32 alone would cost |x| roundings.
@@ -103,7 +111,7 @@ template <bool OUT>
 __global__ __launch_bounds__(256) void k_dn_chunk_prep(
     int t, int heads, int qk_heads, int dv, int nch, const float* __restrict__ q,
     const float* __restrict__ k, const float* __restrict__ v, const float* __restrict__ g,
-    const float* __restrict__ beta, const int64_t* __restrict__ lengths, DnChunkWs ws) {
+    const float* __restrict__ beta, const int64_t* __restrict__ lengths, DnChunkWs ws, int t0) {
   constexpr int C = kDnChunk, DK = kDnChunkDk;
   __shared__ __attribute__((aligned(16))) float kk[C][kDnKkRow];
   __shared__ __attribute__((aligned(16))) float qk[OUT ? C : 1][kDnKkRow];
@@ -116,7 +124,7 @@ __global__ __launch_bounds__(256) void k_dn_chunk_prep(
   id /= nch;
   const int kh = id % qk_heads, row = id / qk_heads;
   const int rep = heads / qk_heads;
-  const int n = dn_steps(lengths, row, t);
+  const int n = dn_steps(lengths, row, t, t0);
   const int c0 = ch * C;
   if (c0 >= n) return;  // uniform: the scan does not visit this chunk
   const int tid = threadIdx.x, w = uniform(tid / kWave), lane = tid & (kWave - 1);
@@ -315,7 +323,7 @@ template <bool OUT, bool COMMIT>
 __global__ __launch_bounds__(256 * kDnScanTiles, 2) void k_dn_chunk_scan(
     float* __restrict__ state, int64_t slots_total, const int64_t* __restrict__ slot, int t,
     int heads, int qk_heads, int dv, int nch, const float* __restrict__ v,
-    const int64_t* __restrict__ lengths, float* __restrict__ out, DnChunkWs ws, int bhs) {
+    const int64_t* __restrict__ lengths, float* __restrict__ out, DnChunkWs ws, int bhs, DnPiece piece) {
   constexpr int C = kDnChunk, DK = kDnChunkDk;
   constexpr int NT = kDnScanTiles;
   __shared__ f32x4_t ss[NT][8 * kWave], sy[NT][4 * kWave], su[NT][4 * kWave], sd[NT][4 * kWave];
@@ -326,7 +334,7 @@ __global__ __launch_bounds__(256 * kDnScanTiles, 2) void k_dn_chunk_scan(
   const int nt = wave >> 2, w = wave & 3, w2 = 3 - w;
   const int gq = lane >> 4, c = lane & 15;
   const int col = cb * kDnScanCols + 16 * nt + c;
-  const int n = dn_steps(lengths, row, t);
+  const int n = dn_steps(lengths, row, t, piece.t0);
   const int64_t s_idx = slot ? slot[row] : row;
   if (s_idx < 0 || s_idx >= slots_total) {  // no such slot: zero outputs, no state access
     if (OUT && w == 0)
@@ -342,7 +350,9 @@ __global__ __launch_bounds__(256 * kDnScanTiles, 2) void k_dn_chunk_scan(
   const uint32_t vstride = (uint32_t)heads * (uint32_t)dv * 4u;
   const rsrc_t rv = make_rsrc(v + (int64_t)row * t * heads * dv, (uint32_t)n * vstride);
   const rsrc_t ro = make_rsrc(OUT ? out + (int64_t)row * t * heads * dv : v, OUT ? (uint32_t)n * vstride : 0u);
-  float* const sp = state + ((s_idx * heads + head) * DK) * (int64_t)dv + col;
+  float* const pool = state + ((s_idx * heads + head) * DK) * (int64_t)dv + col;
+  float* const kept = piece.carry ? piece.carry + (int64_t)head * DK * dv + col : pool;  // one row
+  const float* const sp = piece.t0 > 0 ? kept : pool;
 
   f32x4_t s[8], own[2];  // every tile of this column tile's S (B operand), and the two it updates
 #pragma unroll
@@ -498,13 +508,14 @@ __global__ __launch_bounds__(256 * kDnScanTiles, 2) void k_dn_chunk_scan(
 #pragma unroll
     for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sp[(int64_t)(16 * (2 * w + m) + 4 * gq + i) * dv] = own[m][i];
+      for (int i = 0; i < 4; ++i) kept[(int64_t)(16 * (2 * w + m) + 4 * gq + i) * dv] = own[m][i];
   }
 }
 
 // Whether (row, head) `bh` has a chunk that the scan left alone.
-__device__ inline bool dn_left_over(const int32_t* odd, int nch, int bh, const int64_t* lengths, int row, int t) {
-  const int used = (dn_steps(lengths, row, t) + kDnChunk - 1) / kDnChunk;
+__device__ inline bool dn_left_over(const int32_t* odd, int nch, int bh, const int64_t* lengths, int row, int t,
+                                    int t0) {
+  const int used = (dn_steps(lengths, row, t, t0) + kDnChunk - 1) / kDnChunk;
   bool any = false;
   for (int i = (int)threadIdx.x; i < used; i += kWave) any |= odd[(int64_t)bh * nch + i] != 0;
   return __ballot(any) != 0ull;

@@ -45,3 +45,11 @@ def test_calls_that_take_the_chunks(need, rows, t, out, heads) -> None:
 def test_shapes_the_chunk_form_does_not_have(need) -> None:
     assert need(1, 1500, True, kd=64) == need(1, 1500, True, vd=96) == need(1, 1500, True, qk=5) == 0
     assert need(1, 65600, True) == 0  # 32-bit offsets inside a row
+
+
+@pytest.mark.parametrize("out", [True, False])
+def test_scratch_of_long_rows_is_bounded(need, out) -> None:
+    """57 KB a step of 64 heads with outputs: a long row goes in pieces, more rows in groups."""
+    assert all(0 < need(1, t, out) <= 256 << 20 for t in (1500, 4608, 4609, 8192, 32768, 65000))
+    assert need(1, 1500, out) < need(4, 1500, out) <= 256 << 20
+    assert need(1, 64, out) < need(1, 65, out)

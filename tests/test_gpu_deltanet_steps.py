@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 import torch
 
+import _mtpk
 import deltanet
 from oracle import deltanet_ref as dn
 
@@ -143,3 +144,91 @@ def test_prep_runs_of_rows(dev, dtype, t, conv_k, kd, vd) -> None:
         tol = 2**-7 if dtype == torch.bfloat16 else 1e-5
         torch.testing.assert_close(x, y, rtol=tol, atol=1e-6)
         assert float(((x - y).abs() > 1e-5 * y.abs() + 1e-6).float().mean()) < 2e-3
+
+
+def _ws_call(state, slots, x, lengths, out, workspace):
+    """`mtpk_delta_rule_ws` with a workspace of the caller's size; its status."""
+    q, k, v, g, beta = x
+    rows, t, qk = q.shape[:3]
+    n, heads, kd, vd = state.shape
+    return _mtpk.lib().mtpk_delta_rule_ws(
+        state.data_ptr(), n, _mtpk.ptr(slots), rows, t, heads, qk, kd, vd, *(y.data_ptr() for y in x), _mtpk.ptr(lengths),
+        _mtpk.ptr(out), workspace.data_ptr(), workspace.numel(), _mtpk.stream_of(state.device))
+
+
+def _need(rows, t, heads, qk, out):
+    return int(_mtpk.lib().mtpk_delta_rule_workspace_bytes(rows, t, heads, qk, 128, 128, int(out)))
+
+
+@pytest.mark.parametrize("with_slots", [True, False])
+@pytest.mark.parametrize("mode", ["verify", "commit", "both"])
+def test_rows_run_in_groups_that_fit(dev, with_slots, mode) -> None:
+    """Three rows in a workspace for two or for one leave the bits of one pass, with a head of the last
+    row that runs step by step; a byte less than one row is refused."""
+    t, heads, qk = 150, 4, 2
+    pool, _, q, k, v, g, beta = _case(21, 5, heads, qk, 128, 128, 3, t)
+    beta[2, 70, 1] = 1.5
+    args = _dev(dev, pool, q, k, v, g, beta)
+    slots = torch.tensor([4, 0, 2], device=dev) if with_slots else None
+    lengths = None if mode == "verify" else torch.tensor([t, 90, 130], device=dev)
+    want_out = mode != "commit"
+    one = _need(1, t, heads, qk, want_out)
+    assert 0 < one and _need(3, t, heads, qk, want_out) == 3 * one
+    seen = []
+    for size in (3 * one, 2 * one, 2 * one + 100, one):
+        state = args[0].clone()
+        out = torch.zeros(3, t, heads, 128, device=dev) if want_out else None
+        ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=dev)  # NaN where nothing was written
+        assert _ws_call(state, slots, args[1:], lengths, out, ws) == 0
+        seen.append((state, out if want_out else state))
+        assert torch.equal(state, seen[0][0]) and torch.equal(seen[-1][1], seen[0][1])
+    assert torch.isfinite(seen[0][1]).all()
+    assert _ws_call(args[0], slots, args[1:], lengths, None if not want_out else seen[0][1], ws[: one - 1]) == _mtpk.EINVAL
+
+
+@pytest.mark.parametrize("mode", ["verify", "commit", "both"])
+def test_a_long_row_runs_in_pieces(dev, mode) -> None:
+    """A row whose scratch passes the bound runs piece after piece with the bits of one pass (which a
+    workspace of the whole row's size still gets); a head with one odd step follows the step-by-step form
+    from the state that the pieces before it left."""
+    t, heads, qk = 4700, 64, 16
+    gen = torch.Generator(device=dev).manual_seed(3)
+    n = lambda *s: torch.randn(*s, generator=gen, device=dev)  # noqa: E731
+    unit = lambda x: x / x.norm(dim=-1, keepdim=True)  # noqa: E731
+    x = [unit(n(1, t, qk, 128)) * 128**-0.5, unit(n(1, t, qk, 128)), n(1, t, heads, 128),
+         -torch.rand(1, t, heads, generator=gen, device=dev), torch.rand(1, t, heads, generator=gen, device=dev)]
+    pool, slots = n(2, heads, 128, 128) * 0.05, torch.tensor([1], device=dev)
+    want_out = mode != "commit"
+    need = _need(1, t, heads, qk, want_out)
+    assert need <= 256 << 20
+
+    def both(length):
+        lengths = None if mode == "verify" else torch.tensor([length], device=dev)
+        res = []
+        for size in (need, 512 << 20):
+            state, out = pool.clone(), torch.zeros(1, t, heads, 128, device=dev) if want_out else None
+            ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=dev)
+            assert _ws_call(state, slots, x, lengths, out, ws) == 0
+            res.append((state, out))
+            if mode == "verify":
+                assert torch.equal(state, pool)
+        assert torch.equal(res[0][0], res[1][0])
+        return res
+
+    for length in (t, 4500, 4000):
+        (_, cut), (_, whole) = both(length)
+        assert not want_out or torch.equal(cut, whole)
+    x[4][0, 4650, 7] = 1.25  # in the last piece: the whole row's form runs this head step by step
+    res = []
+    for size in (need, 512 << 20):
+        state, out = pool.clone(), torch.zeros(1, t, heads, 128, device=dev) if want_out else None
+        ws = torch.full((size,), 0xFF, dtype=torch.uint8, device=dev)
+        assert _ws_call(state, slots, x, None if mode == "verify" else torch.tensor([t], device=dev), out, ws) == 0
+        res.append((state, out))
+    for a, b in zip(*res, strict=True):
+        if a is None:
+            continue
+        a, b = (y[0].transpose(0, 1) if y.shape[1] == t else y[1] for y in (a, b))  # [heads, ...]
+        others = [h for h in range(heads) if h != 7]
+        assert torch.equal(a[others], b[others])
+        _close(a[7].cpu().numpy(), b[7].cpu().numpy())
