@@ -453,11 +453,12 @@ int mtpk_delta_rule(float* state, int64_t slots_total, const int64_t* slot, int6
 /* The same with a workspace for calls of many steps (a prompt's rows): where
  * mtpk_delta_rule_workspace_bytes is positive (k_dim 128, v_dim a multiple of 64, and steps enough
  * for the rows to be the faster form), 64 steps at a time become fp32 matrix products and only every
- * 64th step waits for the state; a (row, head) whose k is longer than 1, whose g is positive, whose beta
- * lies outside [0, 1] or whose v, k, g or beta is not finite runs step by step as before. The bytes are
- * at most 256 MiB: rows run in groups that fit, so that a larger workspace takes fewer launches, and
- * a row that does not fit in pieces of its steps (with that (row, head) step by step in the piece where
- * it occurs). A workspace for one row, or for one row's pieces, is the least. workspace is 256-byte
+ * 64th step waits for the state. A (row, head) runs step by step as before when some step of it has
+ * |k|^2 above 1.01, g that is NaN or positive (-infinity is a decay of zero), beta that is NaN or
+ * outside [0, 1], or a v above 1e30 or not finite; 32 columns of its state do when one of their values
+ * is above 1e30 or not finite. The bytes are at most 256 MiB: rows run in groups that fit, so that a
+ * larger workspace takes fewer launches, and a row that does not fit in pieces of its steps (each
+ * with its own choice of the step-by-step form). A workspace for one row, or for one row's pieces, is the least. workspace is 256-byte
  * aligned. Where the bytes are 0 (always below 16 steps), or with operands that are not 16-byte
  * aligned, the call is mtpk_delta_rule (workspace unused, may be NULL). */
 int64_t mtpk_delta_rule_workspace_bytes(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads,

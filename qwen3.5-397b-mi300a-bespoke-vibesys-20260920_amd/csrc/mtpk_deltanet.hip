@@ -159,12 +159,15 @@ __device__ inline float group_sum(float x) {
   return x;
 }
 
+// `left`, where not null, has a word for each 32 columns of the (row, head) matrices: only those with
+// a nonzero one are written.
 template <int KG, bool OUT, bool COMMIT>
 __device__ __forceinline__ void delta_rule_kg_body(
     int bid, float* __restrict__ state, int64_t slots_total, const int64_t* __restrict__ slot, int t,
     int heads, int rep, int dv, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ g, const float* __restrict__ beta,
-    const int64_t* __restrict__ lengths, float* __restrict__ out, DnPiece piece = {0, nullptr}) {
+    const int64_t* __restrict__ lengths, float* __restrict__ out, DnPiece piece = {0, nullptr},
+    const int32_t* left = nullptr) {
   static_assert(KG == 4 || KG == 8, "row groups of 32 or 16");
   constexpr int DK = 128, QR = DK / KG, CW = 4 * kWave / KG;  // rows per group, columns per wave
   const int nblk = dv / CW;
@@ -175,6 +178,7 @@ __device__ __forceinline__ void delta_rule_kg_body(
   const int col4 = base + 4 * cg;                   // this lane's first state column
   const int64_t s_idx = slot ? slot[row] : row;
   const int64_t o_row = (int64_t)head * dv + col4 + kg;  // kg < 4: the output column it writes
+  const bool writes = !left || left[(int64_t)bh * (dv / kDnScanCols) + col4 / kDnScanCols] != 0;
   if (s_idx < 0 || s_idx >= slots_total) {  // no such slot: zero outputs, no state access
     if (OUT && kg < 4)
       for (int st = 0; st < t; ++st) out[((int64_t)row * t + st) * heads * dv + o_row] = 0.f;
@@ -269,10 +273,10 @@ __device__ __forceinline__ void delta_rule_kg_body(
         const float sum = group_sum<KG>(o[c]);
         if (kg == c) mine = sum;
       }
-      if (kg < 4) out[((int64_t)row * t + st) * heads * dv + o_row] = mine;
+      if (kg < 4 && writes) out[((int64_t)row * t + st) * heads * dv + o_row] = mine;
     }
   }
-  if (COMMIT) {
+  if (COMMIT && writes) {
 #pragma unroll
     for (int i = 0; i < QR; ++i)
       __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_t, s[i]), rsm, (int)voff,
@@ -326,18 +330,18 @@ int launch_delta_rule_mode(float* state, int64_t slots_total, const int64_t* slo
                                             lengths, nullptr, st);
 }
 
-// The (row, head) matrices that the chunk scan left, step by step.
+// The columns that the chunk scan left, step by step: 64 to a workgroup, two of the scan's.
 template <bool OUT, bool COMMIT>
 __global__ __launch_bounds__(kWave, (OUT && COMMIT) ? 2 : 3) void k_delta_rule_rest(
     float* __restrict__ state, int64_t slots_total, const int64_t* __restrict__ slot, int t,
     int heads, int rep, int dv, const float* __restrict__ q, const float* __restrict__ k,
     const float* __restrict__ v, const float* __restrict__ g, const float* __restrict__ beta,
-    const int64_t* __restrict__ lengths, float* __restrict__ out, const int32_t* __restrict__ odd,
-    int nch, DnPiece piece) {
-  const int bh = (int)blockIdx.x / (dv / (4 * kWave / kDnKG));
-  if (!dn_left_over(odd, nch, bh, lengths, bh / heads, t, piece.t0)) return;  // uniform
+    const int64_t* __restrict__ lengths, float* __restrict__ out, const int32_t* __restrict__ left,
+    DnPiece piece) {
+  static_assert(4 * kWave / kDnKG == 2 * kDnScanCols, "");
+  if (!(left[2 * (int64_t)blockIdx.x] | left[2 * (int64_t)blockIdx.x + 1])) return;  // uniform
   delta_rule_kg_body<kDnKG, OUT, COMMIT>((int)blockIdx.x, state, slots_total, slot, t, heads, rep, dv,
-                                         q, k, v, g, beta, lengths, out, piece);
+                                         q, k, v, g, beta, lengths, out, piece, left);
 }
 
 // The scratch of a call: rows run in groups that fit, and a row that does not fit in pieces of whole
@@ -346,10 +350,11 @@ __global__ __launch_bounds__(kWave, (OUT && COMMIT) ? 2 : 3) void k_delta_rule_r
 constexpr int64_t kDnChunkWsBytes = int64_t(256) << 20;
 
 // Workspace of one row's `nch` chunks (a multiple of 256 bytes).
-int64_t dn_chunk_row_bytes(int64_t nch, int64_t heads, int64_t qk_heads, bool want_out) {
+int64_t dn_chunk_row_bytes(int64_t nch, int64_t heads, int64_t qk_heads, int64_t v_dim, bool want_out) {
   const int64_t m = want_out ? 2 : 1;
   return qk_heads * nch * (m + 1) * kDnRowTiles * kDnTile * 4 +
-         heads * nch * (m * kDnSqTiles * kDnTile + 2 * kDnChunk) * 4 + align256(heads * nch * 4);
+         heads * nch * (m * kDnSqTiles * kDnTile + 2 * kDnChunk) * 4 +
+         align256(heads * (nch + v_dim / kDnScanCols) * 4);
 }
 
 // How a call's rows and chunks go into `bytes` of workspace: `rows` rows of `nch` chunks at once, or one
@@ -361,15 +366,15 @@ struct DnPlan {
 };
 DnPlan dn_chunk_plan(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads, int64_t v_dim, bool want_out,
                      int64_t bytes) {
-  const int64_t nch = (t + kDnChunk - 1) / kDnChunk, one = dn_chunk_row_bytes(nch, heads, qk_heads, want_out);
+  const int64_t nch = (t + kDnChunk - 1) / kDnChunk, one = dn_chunk_row_bytes(nch, heads, qk_heads, v_dim, want_out);
   if (one <= bytes) {
     const int64_t fit = std::min(bytes / one, rows);
     return {fit, nch, fit * one, false};
   }
   const int64_t carry = want_out ? align256(heads * kDnChunkDk * v_dim * 4) : 0;
-  const int64_t per = dn_chunk_row_bytes(1, heads, qk_heads, want_out);  // no less than one chunk's share
+  const int64_t per = dn_chunk_row_bytes(1, heads, qk_heads, v_dim, want_out);  // no less than one chunk's share
   const int64_t fit = bytes > carry ? (bytes - carry) / per : 0;
-  return {1, fit, dn_chunk_row_bytes(fit, heads, qk_heads, want_out) + carry, true};
+  return {1, fit, dn_chunk_row_bytes(fit, heads, qk_heads, v_dim, want_out) + carry, true};
 }
 
 // Whether a call's sizes are for the chunk form: its shapes (32-bit byte offsets inside a row), and
@@ -424,6 +429,7 @@ DnChunkWs dn_chunk_ws(void* workspace, int64_t rows, int64_t nch, int64_t heads,
   w.eg = take(slabs * kDnChunk);
   w.dg = take(slabs * kDnChunk);
   w.odd = reinterpret_cast<int32_t*>(p);
+  w.left = w.odd + slabs;
   return w;
 }
 
@@ -447,7 +453,7 @@ int launch_dn_chunks(float* state, int64_t slots_total, const int64_t* slot, int
   if (rc) return rc;
   hipLaunchKernelGGL((k_delta_rule_rest<OUT, COMMIT>), dim3((unsigned)(rows * heads * (dv / (4 * kWave / kDnKG)))),
                      dim3(kWave), 0, st, state, slots_total, slot, (int)t, (int)heads, (int)(heads / qk_heads),
-                     (int)dv, q, k, v, g, beta, lengths, out, ws.odd, (int)nch, piece);
+                     (int)dv, q, k, v, g, beta, lengths, out, ws.left, piece);
   return status_of(hipGetLastError());
 }
 
@@ -860,7 +866,7 @@ int mtpk_delta_rule_ws(float* state, int64_t slots_total, const int64_t* slot, i
     const DnChunkWs ws = dn_chunk_ws(workspace, r, plan.nch, heads, qk_heads, want_out);
     // the carried state lies at the workspace's end
     float* const carry = plan.pieces && !lengths
-        ? reinterpret_cast<float*>(static_cast<char*>(workspace) + dn_chunk_row_bytes(plan.nch, heads, qk_heads, want_out))
+        ? reinterpret_cast<float*>(static_cast<char*>(workspace) + dn_chunk_row_bytes(plan.nch, heads, qk_heads, v_dim, want_out))
         : nullptr;
     const int64_t* const ln = lengths ? lengths + r0 : nullptr;
     float* const stt = slot ? state : state + r0 * heads * k_dim * v_dim;  // no slots: row j is slot j

@@ -15,11 +15,13 @@
 // differenced in fp64: e^(G_i - G_j) of neighbouring steps must not lose the digits that a long
 // chunk's large |G| would cost it in fp32.
 //
-// A masked element is a product with zero there, so a NaN or infinity in one step's row would
-// reach the outputs of earlier steps of its chunk. The prep therefore checks each chunk: finite v,
-// k of at most unit length, g <= 0 and beta in [0, 1] (what the layer produces); a (row, head)
-// with any other chunk is left to the step-by-step form, launched behind the scan, whose workgroups
-// return at once when there is nothing to do.
+// A masked element is a product with zero there, so a NaN or infinity in one step's row, given or by
+// overflow, would reach the outputs of earlier steps of its chunk. The prep therefore checks each
+// chunk (|v| at most kDnLargest, |k|^2 at most 1.01, g <= 0, which takes in -infinity, and beta in [0, 1]:
+// what the layer produces) and the scan the state that it starts from (no value above
+// kDnLargest): then nothing overflows, as k does not lengthen the state and a call has at most 2^22
+// steps. A (row, head) with any other chunk, or 32 columns with any other state, are left to the step-by-step
+// form, launched behind the scan, whose workgroups return at once when there is nothing to do.
 #pragma once
 
 #include "mtpk_device.h"
@@ -30,6 +32,7 @@ constexpr int kDnChunk = 64;      // steps per chunk (C)
 constexpr int kDnChunkDk = 128;   // the only k_dim of this form
 constexpr int kDnScanCols = 32;   // state columns per scan workgroup
 constexpr int kDnScanTiles = kDnScanCols / 16;
+constexpr float kDnLargest = 1e30f;  // of v and of the first state; the sums of 2^22 steps of it are finite
 constexpr int kDnKkRow = kDnChunk + 4;  // LDS row of a 64 x 64 matrix, padded
 
 __device__ inline f32x4_t mfma16x16x4(float a, float b, f32x4_t c) {
@@ -43,7 +46,8 @@ __device__ inline f32x4_t mfma16x16x4(float a, float b, f32x4_t c) {
 // [4 step tiles][8], q the same (calls with outputs) and k transposed [8 k_dim tiles][4]; per (row,
 // head, chunk): T [4][4], the masked q . k [4][4] (calls with outputs; both lower triangular, the
 // tiles above the diagonal are not written), e^(G_i) and e^(G_C - G_i) [64] each, and a word that
-// is nonzero when the chunk is not for this form.
+// is nonzero when the chunk is not for this form. Per (row, head, scan workgroup): a word that is
+// nonzero when the scan left its columns.
 struct DnChunkWs {
   float* kr;
   float* qr;   // null without outputs
@@ -53,6 +57,7 @@ struct DnChunkWs {
   float* eg;
   float* dg;
   int32_t* odd;
+  int32_t* left;
 };
 constexpr int kDnTile = 256;                  // floats of a tile
 constexpr int kDnRowTiles = 32, kDnSqTiles = 16;  // tiles of a [64][128] and of a [64][64] matrix
@@ -292,15 +297,16 @@ __global__ __launch_bounds__(256) void k_dn_chunk_prep(
 #pragma unroll
       for (int rt = ct; rt < 4; ++rt) tm[(rt * 4 + ct) * kWave + lane] = dn_mma(tt[rt][ct], one, zero) * bc;
     }
-    float bad = 0.f;  // stays 0, or NaN once a value is not finite
+    uint32_t most = 0;  // bits of the largest |v|; NaN and infinity lie above every number
     for (int d = 0; d < dv; d += kWave) {
       if (d > 0) load_v(v0, d);
 #pragma unroll
       for (int e = 0; e < kAhead; ++e)
 #pragma unroll
-        for (int x = 0; x < 4; ++x) bad = fmaf(bits_f32(v0[e][x]), 0.f, bad);
+        for (int x = 0; x < 4; ++x) most = max(most, v0[e][x] & 0x7fffffffu);
     }
-    const bool fine = gl <= 0.f && bl >= 0.f && bl <= 1.f && kk[lane][lane] <= 1.01f && bad == 0.f;
+    const bool fine =
+        gl <= 0.f && bl >= 0.f && bl <= 1.f && kk[lane][lane] <= 1.01f && most <= f32_bits(kDnLargest);
     const bool odd = __ballot(fine) != ~0ull;
     if (lane == 0) ws.odd[slab] = odd;
     own_lds();
@@ -327,6 +333,7 @@ __global__ __launch_bounds__(256 * kDnScanTiles, 2) void k_dn_chunk_scan(
   constexpr int C = kDnChunk, DK = kDnChunkDk;
   constexpr int NT = kDnScanTiles;
   __shared__ f32x4_t ss[NT][8 * kWave], sy[NT][4 * kWave], su[NT][4 * kWave], sd[NT][4 * kWave];
+  __shared__ int over[4 * NT];
   // the column blocks of one head are bhs apart: with bhs a multiple of 8 they share an XCD's L2
   const int bh = blockIdx.x % bhs, cb = blockIdx.x / bhs;
   const int row = bh / heads, head = bh - row * heads, kh = head / (heads / qk_heads);
@@ -336,16 +343,22 @@ __global__ __launch_bounds__(256 * kDnScanTiles, 2) void k_dn_chunk_scan(
   const int col = cb * kDnScanCols + 16 * nt + c;
   const int n = dn_steps(lengths, row, t, piece.t0);
   const int64_t s_idx = slot ? slot[row] : row;
+  int32_t* const left = ws.left + (int64_t)bh * (dv / kDnScanCols) + cb;
   if (s_idx < 0 || s_idx >= slots_total) {  // no such slot: zero outputs, no state access
     if (OUT && w == 0)
       for (int st = gq; st < t; st += 4) out[(((int64_t)row * t + st) * heads + head) * dv + col] = 0.f;
+    if (tid == 0) *left = 0;
     return;  // uniform over the workgroup
   }
   const int used = (n + C - 1) / C;
   const int64_t slab0 = (int64_t)bh * nch;
   bool odd = false;
   for (int i = lane; i < used; i += kWave) odd |= ws.odd[slab0 + i] != 0;
-  if (__ballot(odd) != 0ull || used == 0) return;  // uniform: the step-by-step form takes it
+  const bool given = __ballot(odd) != 0ull;  // uniform: the step-by-step form takes it
+  if (given || used == 0) {
+    if (tid == 0) *left = given;
+    return;
+  }
 
   const uint32_t vstride = (uint32_t)heads * (uint32_t)dv * 4u;
   const rsrc_t rv = make_rsrc(v + (int64_t)row * t * heads * dv, (uint32_t)n * vstride);
@@ -419,12 +432,25 @@ __global__ __launch_bounds__(256 * kDnScanTiles, 2) void k_dn_chunk_scan(
   ring_fence();
   load_cols(0);
   ring_fence();
+  uint32_t most = 0;
+#pragma unroll
+  for (int m = 0; m < 8; ++m)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) most = max(most, f32_bits(s[m][i]) & 0x7fffffffu);
+  const bool large = __ballot(most > f32_bits(kDnLargest)) != 0ull;
+  if (lane == 0) over[wave] = large;
   auto barrier = [&]() {  // LDS only: the next chunk's loads stay in flight
     ring_fence();
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();
     ring_fence();
   };
+  barrier();
+  int any = 0;
+#pragma unroll
+  for (int i = 0; i < 4 * NT; ++i) any |= over[i];
+  if (tid == 0) *left = any;
+  if (any) return;  // uniform over the workgroup
   int ch = 0;  // used >= 1: a bottom-tested loop keeps the loads above in front of it
 #pragma clang loop unroll(disable)
   do {
@@ -510,15 +536,6 @@ __global__ __launch_bounds__(256 * kDnScanTiles, 2) void k_dn_chunk_scan(
 #pragma unroll
       for (int i = 0; i < 4; ++i) kept[(int64_t)(16 * (2 * w + m) + 4 * gq + i) * dv] = own[m][i];
   }
-}
-
-// Whether (row, head) `bh` has a chunk that the scan left alone.
-__device__ inline bool dn_left_over(const int32_t* odd, int nch, int bh, const int64_t* lengths, int row, int t,
-                                    int t0) {
-  const int used = (dn_steps(lengths, row, t, t0) + kDnChunk - 1) / kDnChunk;
-  bool any = false;
-  for (int i = (int)threadIdx.x; i < used; i += kWave) any |= odd[(int64_t)bh * nch + i] != 0;
-  return __ballot(any) != 0ull;
 }
 
 }  // namespace mtpk

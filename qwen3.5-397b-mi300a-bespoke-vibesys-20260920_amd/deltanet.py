@@ -83,8 +83,9 @@ def commit(state: torch.Tensor, conv_state: torch.Tensor, slots: torch.Tensor, q
            k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, beta: torch.Tensor,
            lengths: torch.Tensor, proj: torch.Tensor, idx: torch.Tensor, channels: int) -> None:
     """`delta_rule(state, slots, q, k, v, g, beta, lengths, want_out=False)` and
-    `conv_commit(conv_state, slots, proj, idx, channels)` as one launch where the layer's sizes
-    allow it (`mtpk_deltanet_commit`); same arguments, same results."""
+    `conv_commit(conv_state, slots, proj, idx, channels)`, same arguments, same results: one launch
+    where the layer's sizes allow it (`mtpk_deltanet_commit`), and over many steps the rule's own
+    launches, then the window's (`mtpk_deltanet_commit_ws`)."""
     device = _mtpk.require_device(state, conv_state, slots, q, k, v, g, beta, lengths, proj, idx)
     if state.dtype != torch.float32 or state.dim() != 4 or not state.is_contiguous():
         raise ValueError("state must be a contiguous f32 [slots, heads, k_dim, v_dim] tensor")

@@ -60,7 +60,7 @@ def test_rows_without_slots_and_bad_slots(dev) -> None:
     assert not out[1:].any()
 
 
-@pytest.mark.parametrize("what", ["beta", "long_k", "growing", "inf_v", "nan_v", "nan_k", "minus_inf_g"])
+@pytest.mark.parametrize("what", ["beta", "long_k", "growing", "inf_v", "nan_v", "nan_k", "minus_inf_g", "overflow"])
 def test_heads_outside_the_chunk_form_run_step_by_step(dev, what) -> None:
     """One head of one row breaks the chunk form's terms at step 70 of 100: it gets what the
     step-by-step form gives (bit for bit; NaN only from that step on), the others are unchanged."""
@@ -75,6 +75,10 @@ def test_heads_outside_the_chunk_form_run_step_by_step(dev, what) -> None:
         g[1, 70, 2] = 0.25
     elif what == "minus_inf_g":
         g[1, 70, 2] = -np.inf  # a decay of exactly zero is the chunk form's too
+    elif what == "overflow":  # finite values whose update at step 71 is not
+        k[1, 71, 2] = k[1, 70, 2]
+        beta[1, 70:72, 2], g[1, 71, 2] = 1, 0
+        v[1, 70, 2, 5], v[1, 71, 2, 5] = 3e38, -3e38
     else:
         (v if what.endswith("v") else k)[1, 70, 2, 5] = np.inf if what == "inf_v" else np.nan
     args = _dev(dev, pool, slots.astype(np.int64), q, k, v, g, beta)
@@ -158,6 +162,33 @@ def _ws_call(state, slots, x, lengths, out, workspace):
 
 def _need(rows, t, heads, qk, out):
     return int(_mtpk.lib().mtpk_delta_rule_workspace_bytes(rows, t, heads, qk, 128, 128, int(out)))
+
+
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan, 3e38])
+def test_a_state_outside_the_chunk_form_runs_step_by_step(dev, value) -> None:
+    """A column of one head's state is not finite, or too large to sum: its 32 columns get the bits of the
+    step-by-step form, all others the chunks', in the outputs and in the advanced state."""
+    pool, slots, q, k, v, g, beta = _case(7, 4, 4, 4, 128, 128, 2, 100)
+    args = _dev(dev, pool, slots.astype(np.int64), q, k, v, g, beta)
+    n, t10 = torch.full((2,), 100, device=dev), torch.full((2,), 10, device=dev)
+    plain_state = args[0].clone()
+    plain = deltanet.delta_rule(plain_state, *args[1:], n)
+    args[0][int(slots[1]), 2, 9, 40] = float(value)
+    state = args[0].clone()
+    got = deltanet.delta_rule(state, *args[1:], n)
+    assert torch.equal(deltanet.delta_rule(*args).view(torch.int32), got.view(torch.int32))  # verify: the same
+    p, piece = args[0].clone(), []
+    for s in range(0, 100, 10):
+        piece.append(deltanet.delta_rule(p, args[1], *(x[:, s : s + 10].contiguous() for x in args[2:]), t10))
+    steps, mine, cols = torch.cat(piece, dim=1), (1, slice(None), 2), slice(32, 64)
+    same = lambda a, b: torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num())  # noqa: E731
+    assert same(got[mine][:, cols], steps[mine][:, cols])
+    assert same(state[int(slots[1]), 2, :, cols], p[int(slots[1]), 2, :, cols])
+    assert not torch.equal(got[mine][:, cols], plain[mine][:, cols])
+    for a, b, at in ((got, plain, mine), (state, plain_state, (int(slots[1]), 2))):
+        a, b = a.clone(), b.clone()
+        a[at][..., cols] = b[at][..., cols] = 0
+        assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("with_slots", [True, False])
