@@ -207,6 +207,17 @@ int mtpk_fused_moe_shared(const void* x, int x_dtype, int64_t tokens, int64_t hi
                           int gate_dtype, int64_t gate_stride, void* workspace,
                           int64_t workspace_bytes, void* out, void* stream);
 
+/* mtpk_fused_moe_shared with the number of experts that the routing names, this shard's and all others'
+ * (0: not known). It changes no value, only the choice of kernels: every shard sees every assignment,
+ * and a prompt's rows take 64-token work units where a shard's share of them is large enough. */
+int mtpk_fused_moe_of(const void* x, int x_dtype, int64_t tokens, int64_t hidden, const uint8_t* gate_up,
+                      const uint8_t* gate_up_scale, const uint8_t* down, const uint8_t* down_scale,
+                      int64_t local_experts, int64_t inter_dim, const void* a_expert, int expert_dtype,
+                      const void* a_weight, int weight_dtype, int top_k, int expert_lo, int expert_hi,
+                      int64_t total_experts, const void* shared, int shared_dtype, const void* shared_gate,
+                      int gate_dtype, int64_t gate_stride, void* workspace, int64_t workspace_bytes, void* out,
+                      void* stream);
+
 /* `mtpk_fused_moe_shared` without a workspace argument: its scratch (work list, intermediate
  * planes, y) is the library's own file-scope device buffer of MTPK_MOE_STATIC_SCRATCH bytes, one
  * per GPU, held until the process ends. Nothing is allocated, so the call suits code that cannot

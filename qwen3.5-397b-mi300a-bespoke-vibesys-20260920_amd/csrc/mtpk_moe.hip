@@ -9,13 +9,15 @@
 //               as bf16 hi/lo planes (16 significant bits)
 //     down      per (unit, 64 hidden rows): same decode, MFMA over both planes; fp32 y
 //     combine   per token: sum of weight * y over its top_k assignments in j order
-//     From 14 assignments per expert the units hold up to 64 tokens (mtpk_moe_wide.h).
+//     Where a prompt leaves enough live assignments (wide_min_live) the units hold up to 64 tokens
+//     (mtpk_moe_wide.h).
 //   direct path (tokens <= 4): gate_up with one unit per assignment (no prep), then a
 //     per-token down that also combines (no y, no combine launch)
 // Each wave keeps a ring of trips (weight + activation loads) in flight ahead of the MFMAs.
 // The weight stream is the only HBM-sized traffic; nothing dequantised is ever stored.
 // Lane mapping and K coverage of one MFMA tile: see mtpk_common.h ("MoE lane mapping").
 
+#include <algorithm>
 #include <mutex>
 #include <type_traits>
 
@@ -2018,19 +2020,29 @@ UnitSrc unit_direct(const void* a_expert, int edt, const void* a_weight, int wdt
 }
 
 // Wide units (mtpk_moe_wide.h): bf16 rows of the LDS kernels' K ranges, offsets below 2^31 (bit 31
-// marks a load that is not made), from kWideMinPerExpert assignments per local expert. Below it most
-// units hold a tile of 16 tokens either way, and the 16-token kernels, with their stores held back
-// and items pipelined, stream weights faster. 512 experts, top-10, Zipf(1.1), 16-token units against
-// wide ones: 256 rows (5 per expert) 539 / 579 us, 400 (8) 660 / 677, 600 (12) 803 / 797, 1024 (20)
-// 1047 / 929, 2048 (40) 1604 / 1259. How many assignments are live is known only to the prep (a shard
-// of the experts sees every token's): the host takes these launches when there can be enough, the
-// prep chooses, and the other form's two launches find no unit (a few us).
-constexpr int64_t kWideMinPerExpert = 14;
-bool wide_units(int64_t tokens, int64_t hidden, int64_t inter_dim, int64_t local_experts, int64_t a) {
+// marks a load that is not made), from wide_min_live live assignments. Two things set it. Below about 12
+// per local expert most units hold a tile of 16 tokens either way, and the 16-token kernels, with their
+// stores held back and items pipelined, stream weights faster; and with few experts their wide units
+// alone do not fill the chip's 512 workgroups a few times over. Top-10, 16-token units / wide ones, us
+// (live per expert): 512 experts, Zipf(1.1), (10) 768 / 798, (14) 888 / 855, (24) 1166 / 1010, (40) 1604 /
+// 1259; 256 (14) 444 / 455, (18) 503 / 494, (32) 701 / 583; 128 (14) 240 / 244, (24) 296 / 298, (32) 363 /
+// 305, evenly spread (18) 261 / 225; 64 (24) 158 / 178, (32) 191 / 178, (48) 249 / 203; 32 (32) 100 / 107,
+// (48) 134 / 112. 1024 + 12 per expert is 14, 16, 20, 28 and 44 per expert of 512, 256, 128, 64 and 32.
+//
+// How many assignments are live is known only to the prep, which chooses, and the other form's two
+// launches then find no unit: 5-6 us, which is 5 to 10 % of a small shard's call. A shard of the experts
+// sees every token's assignments, so the host makes the wide launches only when the local experts' even
+// share of them is enough, of all experts where the caller names their number, else of 512 (or
+// as many as the range shows there to be).
+constexpr int64_t wide_min_live(int64_t local_experts) { return 1024 + 12 * local_experts; }
+constexpr int64_t kExpertsAssumed = 512;
+bool wide_units(int64_t tokens, int64_t hidden, int64_t inter_dim, int64_t local_experts, int64_t expert_hi,
+                int64_t total_experts, int64_t a) {
   constexpr int64_t lim = int64_t(1) << 31;
-  return a >= kWideMinPerExpert * local_experts && tokens > kDirectMaxTokens && hidden % 512 == 0 &&
-         hidden <= 4096 && inter_dim % 512 == 0 && inter_dim <= 1024 && tokens * hidden * 2 < lim &&
-         a * inter_dim * 4 < lim;
+  const int64_t all = std::max(total_experts > 0 ? total_experts : kExpertsAssumed, expert_hi);
+  return a * local_experts >= wide_min_live(local_experts) * all && tokens > kDirectMaxTokens &&
+         hidden % 512 == 0 && hidden <= 4096 && inter_dim % 512 == 0 && inter_dim <= 1024 &&
+         tokens * hidden * 2 < lim && a * inter_dim * 4 < lim;
 }
 
 template <bool UP>
@@ -2290,6 +2302,19 @@ int mtpk_fused_moe_shared(const void* x, int x_dtype, int64_t tokens, int64_t hi
                           const void* shared, int shared_dtype, const void* shared_gate,
                           int gate_dtype, int64_t gate_stride, void* workspace,
                           int64_t workspace_bytes, void* out, void* stream) {
+  return mtpk_fused_moe_of(x, x_dtype, tokens, hidden, gate_up, gate_up_scale, down, down_scale,
+                           local_experts, inter_dim, a_expert, expert_dtype, a_weight, weight_dtype, top_k,
+                           expert_lo, expert_hi, 0, shared, shared_dtype, shared_gate, gate_dtype,
+                           gate_stride, workspace, workspace_bytes, out, stream);
+}
+
+int mtpk_fused_moe_of(const void* x, int x_dtype, int64_t tokens, int64_t hidden, const uint8_t* gate_up,
+                      const uint8_t* gate_up_scale, const uint8_t* down, const uint8_t* down_scale,
+                      int64_t local_experts, int64_t inter_dim, const void* a_expert, int expert_dtype,
+                      const void* a_weight, int weight_dtype, int top_k, int expert_lo, int expert_hi,
+                      int64_t total_experts, const void* shared, int shared_dtype, const void* shared_gate,
+                      int gate_dtype, int64_t gate_stride, void* workspace, int64_t workspace_bytes, void* out,
+                      void* stream) {
   if (!x || !out || !workspace || !dtype_float_ok(x_dtype)) return MTPK_EINVAL;
   if (shared && (!shared_gate || !dtype_float_ok(shared_dtype) || !dtype_float_ok(gate_dtype) ||
                  gate_stride < 0))
@@ -2342,7 +2367,7 @@ int mtpk_fused_moe_shared(const void* x, int x_dtype, int64_t tokens, int64_t hi
   }
   if (xp == 1 && aligned16(x) && aligned16(gate_up) && aligned16(down) &&
       gemm_shapes_ok(hidden, inter_dim, local_experts) &&
-      wide_units(tokens, hidden, inter_dim, local_experts, a)) {
+      wide_units(tokens, hidden, inter_dim, local_experts, expert_hi, total_experts, a)) {
     const hipStream_t hs = (hipStream_t)stream;
     if (!a_expert || !a_weight || !gate_up_scale || !down_scale || !dtype_index_ok(expert_dtype) ||
         !dtype_float_ok(weight_dtype))
@@ -2353,7 +2378,7 @@ int mtpk_fused_moe_shared(const void* x, int x_dtype, int64_t tokens, int64_t hi
     const int64_t plane = a * inter_dim;
     hipLaunchKernelGGL(k_moe_prep_wide, dim3(1), dim3(kPrepThreads), 0, hs, a_expert, expert_dtype,
                        a_weight, weight_dtype, (int)a, expert_lo, (int)local_experts, sorted, units,
-                       (int)mu, n_units, kWideMinPerExpert * local_experts);
+                       (int)mu, n_units, wide_min_live(local_experts));
     rc = launch_wide<true>(xplanes, tokens * hidden, 0, (int)hidden, gate_up, gate_up_scale,
                            (int)inter_dim, src, top_k, inter, plane, nullptr, hs);
     if (rc) return rc;

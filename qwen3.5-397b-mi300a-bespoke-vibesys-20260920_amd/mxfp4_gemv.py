@@ -214,12 +214,15 @@ def fused_moe(
     A smaller one, such as the reference's `[max_batch * top_k, intermediate]`, or none, takes a
     grow-only workspace kept per (device, stream): no allocation once it has reached the
     largest size used. Under graph capture the call allocates its own, once, for the graph.
-    `order`, `grouped` and `total_experts` are accepted for signature compatibility: the work
-    list groups assignments by expert at every width, so there is nothing for them to select.
+    `total_experts` is the number that the routing names, this shard's and all others'; it
+    changes no value, only when a prompt's rows take 64-token work units (without it a shard of
+    512 is assumed). `order` and `grouped` are accepted for signature compatibility: the work list
+    groups assignments by expert at every width, so there is nothing for them to select.
     """
     _validate(x, experts, routing, top_k)
     a_expert, a_weight = routing
     lo, hi = expert_range
+    total = total_experts if isinstance(total_experts, int) and 0 < total_experts < 2**31 else 0
     device = _mtpk.require_device(x, a_expert, a_weight, experts["gate_up"])
     tokens, hidden = x.shape
     gate_up, down = experts["gate_up"], experts["down"]
@@ -248,16 +251,16 @@ def fused_moe(
         gate_ptr, gate_code, gate_stride = (shared_gate.data_ptr(), _mtpk.float_code(shared_gate.dtype),
                                             shared_gate.stride(0))
     _mtpk.check(
-        lib.mtpk_fused_moe_shared(
+        lib.mtpk_fused_moe_of(
             x.data_ptr(), xcode, tokens, hidden,
             gate_up.data_ptr(), experts["gate_up_scale"].data_ptr(),
             down.data_ptr(), experts["down_scale"].data_ptr(), local, intermediate,
             a_expert.data_ptr(), _mtpk.index_code(a_expert.dtype),
             a_weight.data_ptr(), _mtpk.float_code(a_weight.dtype),
-            top_k, lo, hi, sh_ptr, sh_code, gate_ptr, gate_code, gate_stride,
+            top_k, lo, hi, total, sh_ptr, sh_code, gate_ptr, gate_code, gate_stride,
             ws.data_ptr(), ws.numel() * ws.element_size(), out.data_ptr(), _mtpk.stream_of(device),
         ),
-        "mtpk_fused_moe_shared",
+        "mtpk_fused_moe_of",
     )  # fmt: skip
     return out
 

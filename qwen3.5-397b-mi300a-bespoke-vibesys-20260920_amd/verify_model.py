@@ -654,8 +654,8 @@ class Model:
         elif mxfp4_gemv.available(h.device):
             # the shared expert's gated term is added inside the routed layer's combine
             return mxfp4_gemv.fused_moe(h.contiguous(), w["experts"], assign, c.top_k, (0, c.experts),
-                                        inter=self.moe_ws, shared=shared.contiguous(),
-                                        shared_gate=routing[:, c.experts :])
+                                        inter=self.moe_ws, total_experts=c.experts,
+                                        shared=shared.contiguous(), shared_gate=routing[:, c.experts :])
         else:
             # SEED_FUSED_MOE=0 (or the CPU): the torch dequant-then-multiply path of
             # `_routed_grouped` (`model.py:3170-3236`), dequantised by the torch table lookup
