@@ -2053,7 +2053,7 @@ int launch_wide(const uint16_t* x, int64_t x_elems, int64_t x_plane, int K, cons
   auto kern = k_moe_wide<UP>;
   if (occ == 0) occ = occupancy_per_cu(kern, kWideThreads);
   constexpr int tiles = UP ? kWideWaves : 4 * kWideWaves;
-  const int64_t items = (int64_t)src.max_units * (((N >> 4) + tiles - 1) / tiles);
+  const int64_t items = (int64_t)src.max_units * (N / (16 * tiles));
   const int64_t cap = (int64_t)device_cu_count() * occ;
   hipLaunchKernelGGL(kern, dim3((unsigned)(items < cap ? items : cap)), dim3(kWideThreads), 0, st, x,
                      (uint32_t)(x_elems * 2), x_plane, K, wq, ws, N, src, top_k, inter, inter_plane, y);

@@ -10,7 +10,8 @@
 //   down     item = (half a unit, 512 hidden rows); a wave has four tiles of 16 rows. Two planes
 //            make a staged row twice as long, and four tiles of 64 tokens would spill.
 // Measured at 2048 rows: gate_up 671 us, down 519 us, the whole call 1604 -> 1259 us. The sums run in
-// the 16-token kernels' order: the same bits.
+// the order of k_moe_gate_up_lds and k_moe_down_lds: the same bits (not k_moe_gate_up's split form,
+// which takes calls of few units). N is a multiple of 512: every item has all of its weight rows.
 // What bounds it is the weight stream as long as most experts have one unit. Token rows go straight
 // to LDS (256 k a chunk, no registers), so that 128 VGPRs leave two workgroups a CU and one's item
 // start hides behind the other's stream. The weights are the A operand: a lane ends with
@@ -48,7 +49,7 @@ __global__ __launch_bounds__(kWideThreads, 4) void k_moe_wide(
   constexpr int kItemTiles = UP ? kWideWaves : kWideWaves * S;
   static_assert(S * 16 * kTurns * 16 * kWideWaves <= kWideBuf, "layout");
   __shared__ __attribute__((aligned(16))) uint8_t xs[2 * kWideBuf];
-  const int ntile = N >> 4, ngroup = (ntile + kItemTiles - 1) / kItemTiles;
+  const int ngroup = N / (16 * kItemTiles);
   const int n_items = min(sload(src.n_units, 0), src.max_units) * ngroup * kHalves;
   const int tid = threadIdx.x, wave = uniform(tid / kWave);
   const int nb = K >> 5, ntrip = nb >> 2, nchunk = ntrip / TPC, segs = nb >> 4;
@@ -79,9 +80,7 @@ __global__ __launch_bounds__(kWideThreads, 4) void k_moe_wide(
     const int tile0 = UP ? q * kWideWaves + wave : (q * kWideWaves + wave) * S;
     const rsrc_t rw = make_rsrc(wq + (int64_t)e * exp_bytes, exp_bytes);
     const rsrc_t rs = make_rsrc(ws + (int64_t)e * rows * nb, (uint32_t)rows * (uint32_t)nb);
-    auto stream_row = [&](int r) {  // first row of stream r, clamped into the expert's rows
-      return UP ? r * N + min(tile0, ntile - 1) * 16 : min(tile0 + r, ntile - 1) * 16;
-    };
+    auto stream_row = [&](int r) { return UP ? r * N + tile0 * 16 : (tile0 + r) * 16; };  // first row of stream r
 
     auto run = [&](auto nt_c) {
       constexpr int NT = decltype(nt_c)::value;  // token tiles of this unit
@@ -228,7 +227,6 @@ __global__ __launch_bounds__(kWideThreads, 4) void k_moe_wide(
         if (16 * t + out.c >= cnt) continue;
         const int64_t om = src.sorted[first + 16 * t + out.c];
         if (UP) {
-          if (tile0 >= ntile) continue;
           uint16_t hi[4], lo[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
@@ -242,8 +240,7 @@ __global__ __launch_bounds__(kWideThreads, 4) void k_moe_wide(
         } else {
 #pragma unroll
           for (int r = 0; r < S; ++r)
-            if (tile0 + r < ntile)
-              *reinterpret_cast<f32x4_t*>(y + om * N + (tile0 + r) * 16 + 4 * out.g) = acc[r][t];
+            *reinterpret_cast<f32x4_t*>(y + om * N + (tile0 + r) * 16 + 4 * out.g) = acc[r][t];
         }
       }
     };
