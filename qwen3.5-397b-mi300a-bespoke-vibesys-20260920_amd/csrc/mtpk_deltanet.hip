@@ -468,15 +468,14 @@ int launch_dn_chunks(float* state, int64_t slots_total, const int64_t* slot, int
 // loaded once for the R rows that see it, all R + conv_k - 1 at once, instead of once per row and
 // tap. The last workgroups write g and beta, a thread per (row, head).
 //
-// 30.8 us at 1500 rows of 12288 channels (111 MB: 3.6 TB/s; the exponentials and divisions of 18 M
-// SiLUs come next) and 8.2 us at 192; a wave per (row, unit) with 16-bit loads took 118 and 21 us.
+// 30 us at 1500 rows of 12288 channels (111 MB: 3.7 TB/s; the exponentials and divisions of 18 M
+// SiLUs come next) and 7.2 us at 192; a wave per (row, unit) with 16-bit loads took 114 and 19 us.
 //
 // Conv taps run in order j = 0 .. conv_k - 1 as separate products and sums (no fused
 // multiply-add), as the torch form does them.
 constexpr int kPrepThreadsDn = 256;
 constexpr int kConvMaxK1 = 8;  // conv_k - 1 at most
 constexpr int kPrepMaxDim = 256;  // widest head
-constexpr int kPrepRows = 8;  // rows a wave takes (4 for calls of at most 4 steps)
 
 struct DnPrepArgs {
   const void* proj;       // [B * t, proj_stride] model dtype: qkv (C), z, b (vh), a (vh)
@@ -643,17 +642,108 @@ __global__ __launch_bounds__(kPrepThreadsDn) void k_deltanet_prep(DnPrepArgs a) 
   }
 }
 
-template <int K, bool PAIR, int NI>
+// The same, a wave per (verify row, head unit): lane l holds channels l, l + 64, ..., every column is
+// loaded for each row and tap that sees it, and a workgroup takes 4 units of one row (grid: rows x
+// units / 4; that of unit group 0 also writes the row's g and beta).
+__global__ __launch_bounds__(kPrepThreadsDn) void k_deltanet_prep_rows(DnPrepArgs a) {
+  const int rs = blockIdx.x;  // b * t + s
+  const int b = rs / a.t, s = rs - b * a.t;
+  const int tid = threadIdx.x, wave = tid / kWave, lane = tid & (kWave - 1);
+  const int k1 = a.conv_k - 1;
+  const int C = 2 * a.kh * a.kd + a.vh * a.vd;
+  const int64_t slot = a.slot[b];
+  const bool slot_ok = slot >= 0 && slot < a.slots_total;
+  const int units = 2 * a.kh + a.vh;
+  const int u = blockIdx.y * (kPrepThreadsDn / kWave) + wave;
+  if (u < units) {
+    const bool is_v = u >= 2 * a.kh;
+    const int dim = is_v ? a.vd : a.kd;
+    const int c0 = is_v ? 2 * a.kh * a.kd + (u - 2 * a.kh) * a.vd : u * a.kd;
+    float x[kPrepMaxDim / kWave];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < kPrepMaxDim / kWave; ++i) {
+      const int ch = lane + kWave * i;
+      x[i] = 0.f;
+      if (ch >= dim) continue;
+      const int c = c0 + ch;
+      float acc = 0.f;
+#pragma unroll
+      for (int j = 0; j < kConvMaxK1 + 1; ++j) {  // all taps' loads issued together
+        if (j >= a.conv_k) break;
+        const int p = s + j;  // window column: the stored k1, then the t new ones
+        const float win = p < k1 ? (slot_ok ? load_float(a.conv, a.dt, (slot * C + c) * k1 + p) : 0.f)
+                                 : load_float(a.proj, a.dt, ((int64_t)b * a.t + p - k1) * a.proj_stride + c);
+        const float prod = __fmul_rn(win, load_float(a.conv_w, a.dt, (int64_t)c * a.conv_k + j));
+        acc = j == 0 ? prod : __fadd_rn(acc, prod);
+      }
+      float y = acc / (1.f + expf(-acc));
+      if (a.dt == MTPK_BF16) y = bf16_to_f32(f32_to_bf16(y));
+      x[i] = y;
+      ss += y * y;
+    }
+    if (is_v) {
+      float* dst = a.v + ((int64_t)rs * a.vh + (u - 2 * a.kh)) * a.vd;
+#pragma unroll
+      for (int i = 0; i < kPrepMaxDim / kWave; ++i)
+        if (lane + kWave * i < dim) dst[lane + kWave * i] = x[i];
+    } else {
+      const bool is_q = u < a.kh;
+      const float inv = rsqrtf(wave_sum(ss) + a.eps);
+      const float sc = is_q ? a.q_scale : 1.f;
+      float* dst = (is_q ? a.q : a.k) + ((int64_t)rs * a.kh + (is_q ? u : u - a.kh)) * a.kd;
+#pragma unroll
+      for (int i = 0; i < kPrepMaxDim / kWave; ++i)
+        if (lane + kWave * i < dim) dst[lane + kWave * i] = x[i] * inv * sc;
+    }
+  }
+  for (int h = tid; blockIdx.y == 0 && h < a.vh; h += kPrepThreadsDn) {
+    const int64_t base = (int64_t)rs * a.proj_stride + C + a.vh * a.vd;
+    const float braw = load_float(a.proj, a.dt, base + h);
+    const float araw = load_float(a.proj, a.dt, base + a.vh + h);
+    const float x = __fadd_rn(araw, a.dt_bias[h]);
+    const float sp = x > 20.f ? x : log1pf(expf(x));
+    a.beta[(int64_t)rs * a.vh + h] = 1.f / (1.f + expf(-braw));
+    a.g[(int64_t)rs * a.vh + h] = -expf(a.a_log[h]) * sp;
+  }
+}
+
+int launch_deltanet_prep_rows(const DnPrepArgs& a, hipStream_t st) {
+  const int groups = (2 * a.kh + a.vh + kPrepThreadsDn / kWave - 1) / (kPrepThreadsDn / kWave);
+  hipLaunchKernelGGL(k_deltanet_prep_rows, dim3((unsigned)((int64_t)a.B * a.t), (unsigned)groups), dim3(kPrepThreadsDn),
+                     0, st, a);
+  return status_of(hipGetLastError());
+}
+
+template <int K, bool PAIR, int NI, int R>
 int launch_deltanet_prep(DnPrepArgs a, hipStream_t st) {
-  const int R = a.t <= 4 ? 4 : kPrepRows;
   const int64_t waves = (int64_t)a.B * ((a.t + R - 1) / R) * (2 * a.kh + a.vh);
   const int64_t ub = (waves + kPrepThreadsDn / kWave - 1) / (kPrepThreadsDn / kWave);
   const int64_t gb = ((int64_t)a.B * a.t * a.vh + kPrepThreadsDn - 1) / kPrepThreadsDn;
-  if (ub + gb > INT32_MAX) return MTPK_EINVAL;
+  if ((ub + gb) * kPrepThreadsDn > UINT32_MAX) return launch_deltanet_prep_rows(a, st);  // past a grid's threads
   a.unit_blocks = (int)ub;
-  auto kern = R == 4 ? k_deltanet_prep<K, PAIR, NI, 4> : k_deltanet_prep<K, PAIR, NI, kPrepRows>;
-  hipLaunchKernelGGL(kern, dim3((unsigned)(ub + gb)), dim3(kPrepThreadsDn), 0, st, a);
+  hipLaunchKernelGGL((k_deltanet_prep<K, PAIR, NI, R>), dim3((unsigned)(ub + gb)), dim3(kPrepThreadsDn), 0, st, a);
   return status_of(hipGetLastError());
+}
+
+// Rows a wave of the pair form takes: as many as a short call has (rows past the last one are computed
+// for nothing: 64 lanes of one row 7.3 us with 4 rows a wave, 4.7 with one), else 8.
+template <int NI>
+int launch_deltanet_prep_pair(const DnPrepArgs& a, hipStream_t st) {
+  if (a.t == 1) return launch_deltanet_prep<4, true, NI, 1>(a, st);
+  if (a.t == 2) return launch_deltanet_prep<4, true, NI, 2>(a, st);
+  if (a.t <= 4) return launch_deltanet_prep<4, true, NI, 4>(a, st);
+  return launch_deltanet_prep<4, true, NI, 8>(a, st);
+}
+
+// Other types, head dims and windows: runs of 4 rows where they are nearly full and there are many, else a
+// wave per row, whose loads go to more waves at once (in pairs of channels without wide loads, a run
+// needs as many of them, one after another). f32, 16 + 16 + 64 heads of 128, a wave per row / runs of 4:
+// 64 x 1 rows 6.9 / 12.5 us, 48 x 4 17.8 / 12.3, 48 x 5 18.7 / 18.8, 100 10.6 / 8.6, 1500 90 / 55; heads of 64: 100
+// rows 6.0 / 7.2, 300 14 / 11, 1500 54 / 35; 2 + 2 + 4 heads of 16, 300 rows 4.5 / 5.0, 2000 7.7 / 7.3.
+bool deltanet_prep_runs(const DnPrepArgs& a) {
+  const int64_t rows = (int64_t)a.B * a.t, padded = (int64_t)a.B * ((a.t + 3) / 4 * 4);
+  return rows * (2 * a.kh + a.vh) >= 16384 && 4 * padded <= 5 * rows;
 }
 
 // The commit's conv-window update (`deltanet_verify_rollback`, model.py:3907-3972): slot b's
@@ -772,9 +862,9 @@ int mtpk_deltanet_prep(const void* proj, int dtype, int64_t proj_stride, const v
                     ((reinterpret_cast<uintptr_t>(proj) | reinterpret_cast<uintptr_t>(conv_state)) & 3u) == 0 &&
                     aligned16(conv_w) && at8(q) && at8(k) && at8(v);
   const bool wide = k_dim > 128 || v_dim > 128;
-  if (pair && conv_k == 4)
-    return wide ? launch_deltanet_prep<4, true, 2>(a, st) : launch_deltanet_prep<4, true, 1>(a, st);
-  return launch_deltanet_prep<0, false, 2>(a, st);
+  if (pair && conv_k == 4) return wide ? launch_deltanet_prep_pair<2>(a, st) : launch_deltanet_prep_pair<1>(a, st);
+  if (!deltanet_prep_runs(a)) return launch_deltanet_prep_rows(a, st);
+  return wide ? launch_deltanet_prep<0, false, 2, 4>(a, st) : launch_deltanet_prep<0, false, 1, 4>(a, st);
 }
 
 int mtpk_conv_commit(void* conv_state, int dtype, const int64_t* slot, int64_t slots_total,

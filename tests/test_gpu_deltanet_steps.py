@@ -131,11 +131,25 @@ def test_long_commit_is_the_rule_and_the_window(dev) -> None:
     (torch.bfloat16, 25, 9, 128, 128), (torch.float32, 11, 4, 16, 256), (torch.float32, 3, 6, 130, 7),
 ])
 def test_prep_runs_of_rows(dev, dtype, t, conv_k, kd, vd) -> None:
-    """`deltanet.prep` at the edges of its runs of rows, odd head dims and other windows, against the
-    torch chain: sums in the same order, so f32 within a few roundings, and bf16 within the
-    neighbouring value where a SiLU lies at a tie."""
+    """`deltanet.prep` at the edges of its runs of rows, odd head dims and other windows."""
+    _check_prep(dev, dtype, t, conv_k, kd, vd, 2, 4)
+
+
+@pytest.mark.parametrize("dtype,t,conv_k,kd,vd", [
+    (torch.bfloat16, 1, 4, 128, 128), (torch.bfloat16, 2, 4, 64, 130), (torch.bfloat16, 3, 4, 128, 128),
+    # other forms: runs of 4 of many rows (last runs of 3, 1 and 4), and a call whose runs would be half empty
+    (torch.float32, 87, 4, 16, 20), (torch.bfloat16, 85, 9, 33, 130), (torch.bfloat16, 88, 3, 7, 64),
+    (torch.float32, 101, 2, 192, 40), (torch.float32, 5, 4, 16, 20),
+])
+def test_prep_of_many_heads(dev, dtype, t, conv_k, kd, vd) -> None:
+    _check_prep(dev, dtype, t, conv_k, kd, vd, 16, 64)
+
+
+def _check_prep(dev, dtype, t, conv_k, kd, vd, kh, vh) -> None:
+    """Against the torch chain: sums in the same order, so f32 within a few roundings, and bf16 within
+    the neighbouring value where a SiLU lies at a tie."""
     g = torch.Generator().manual_seed(t)
-    b, kh, vh = 2, 2, 4
+    b = 2
     c = 2 * kh * kd + vh * vd
     proj = (torch.randn(b, t, c + vh * vd + 2 * vh, generator=g) * 2).to(dtype).to(dev)
     conv = torch.randn(3, c, conv_k - 1, generator=g).to(dtype).to(dev)
