@@ -51,7 +51,7 @@ def run_counted(x, ex, a_e, a_w, top_k, span, dev, **kw):
 
 
 @pytest.mark.parametrize("hidden,inter", SIZES)
-def test_unit_edges_match_oracle(dev, hidden, inter):
+def test_wide_unit_edges_match_oracle(dev, hidden, inter):
     rng = np.random.default_rng(hidden + inter)
     tokens, top_k, counts = 300, 10, np.zeros(LOCAL, int)
     counts[rng.permutation(LOCAL)[: 4 * len(EDGES)]] = EDGES * 4
@@ -108,4 +108,44 @@ def test_shards_of_experts(dev, tokens, total, named, wide):
     got, units = run_counted(torch.from_numpy(x).to(dev, torch.bfloat16), to_dev(ex, dev), a_e, a_w, top_k, span, dev,
                              total_experts=total if named else None)
     assert (units[0] == 0 and 0 < units[1] < UNSET) if wide else (units[0] > 0 and units[1] == UNSET)
+    assert moe_ref.rel_l2(got.float().cpu().numpy(), want) <= 2e-3
+
+
+# The same counts on 8 experts, too few for wide units: 16-token units of the same sizes.
+@pytest.mark.parametrize("hidden,inter", [(512, 512), (1536, 1024), (4096, 512)])
+@pytest.mark.parametrize("counts", [
+    (15, 16, 17, 31, 32, 33, 47, 48),
+    (49, 63, 64, 65, 1, 0, 128, 130),
+])
+def test_unit_edges_match_oracle(dev, hidden, inter, counts):
+    rng = np.random.default_rng(hidden + inter)
+    tokens, top_k = 131, 5
+    a_e, a_w = routing_with_counts(counts, tokens, top_k, rng)
+    ex = random_experts(len(counts), hidden, inter, seed=3)
+    x = bf16_round(rng.standard_normal((tokens, hidden)).astype(np.float32))
+    want = bf16_round(moe_ref.reference_moe(x, ex, a_e, a_w, top_k, (0, len(counts))))
+    dex, xd = to_dev(ex, dev), torch.from_numpy(x).to(dev, torch.bfloat16)
+    got = run(xd, dex, a_e, a_w, top_k, (0, len(counts)), dev)
+    assert moe_ref.rel_l2(got.float().cpu().numpy(), want) <= 2e-3
+    # 12 tokens at a time take the split-K kernels, whose sums run in another order
+    for t in range(0, tokens, 12):
+        part = slice(t * top_k, min(t + 12, tokens) * top_k)
+        few = run(xd[t : t + 12], dex, np.ascontiguousarray(a_e[part]), np.ascontiguousarray(a_w[part]), top_k,
+                  (0, len(counts)), dev)
+        assert moe_ref.rel_l2(few.float().cpu().numpy(), got[t : t + 12].float().cpu().numpy()) <= 2e-3
+
+
+# The shard's 8 experts see every assignment: 3000 rows of 24 experts leave 1250 of them live per expert,
+# 400 rows of 400 experts 10; 16-token units, as the host sees 8 of 512 experts.
+@pytest.mark.parametrize("tokens,total", [(3000, 24), (400, 400)])
+def test_shard_of_experts_and_long_routing(dev, tokens, total):
+    """More assignments than a prep thread keeps, experts outside the shard, int64 ids."""
+    rng = np.random.default_rng(1)
+    top_k = 10
+    ex = random_experts(8, 512, 512, seed=4)
+    a_e = np.stack([rng.permutation(total)[:top_k] for _ in range(tokens)]).astype(np.int64).reshape(-1)
+    a_w = rng.random(tokens * top_k).astype(np.float32)
+    x = bf16_round(rng.standard_normal((tokens, 512)).astype(np.float32))
+    want = bf16_round(moe_ref.reference_moe(x, ex, a_e, a_w, top_k, (8, 16)))
+    got = run(torch.from_numpy(x).to(dev, torch.bfloat16), to_dev(ex, dev), a_e, a_w, top_k, (8, 16), dev)
     assert moe_ref.rel_l2(got.float().cpu().numpy(), want) <= 2e-3
