@@ -386,7 +386,9 @@ DnPlan dn_chunk_plan(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads, i
 // steps 57 / 68, 64 steps 107 / 69, 65 steps 108 / 113, 128 steps 207 / 116; m = 8, 64 steps 107 / 118,
 // 129 steps 209 / 248, 256 steps 400 / 314; m = 16, 320 steps 643 / 785. Commits: m = 1, 24 steps
 // 26 / 25, 1500 steps 1637 / 116; m = 4, 64 steps 76 / 51, 65 steps 77 / 74; m = 8, 64 steps 81 / 87, 128
-// steps 149 / 131. Near the line the old form keeps the call (the factor 1.05).
+// steps 149 / 131. Near the line the old form keeps the call (the factor
+// 1.03): over 700 measured sizes no choice was the slower one by more than runs differ, and none missed
+// more than a tenth.
 constexpr int64_t kDnChunkMinSteps = 16;  // no call of fewer steps takes the chunk form
 bool dn_chunk_fits(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads, int64_t k_dim, int64_t v_dim,
                    bool want_out) {
@@ -397,15 +399,15 @@ bool dn_chunk_fits(int64_t rows, int64_t t, int64_t heads, int64_t qk_heads, int
   const double m = (double)rows * heads * v_dim / (64 * 128), n = (double)((t + kDnChunk - 1) / kDnChunk);
   double launch, chunk, steps;
   if (want_out) {
-    launch = std::max(20.0, 14 + 10 * std::min(m, 5.0));
+    launch = std::max(20.0, 13 + 10 * std::min(m, 5.0)) - (n == 1 ? 3 * std::clamp(m - 1, 0.0, 4.0) : 0);
     chunk = std::max(5.5, 6.2 * m + 0.18 * m * m);
     steps = 1.5 + 0.75 * m + t * (1.38 + 0.03 * m);
   } else {
-    launch = std::max(19.0, 15 + 5.5 * std::min(m, 7.0));
+    launch = std::max(19.0, 15 + 5.5 * std::min(m, 7.0)) - (n == 1 ? 0.6 * std::clamp(m - 1, 0.0, 4.0) : 0);
     chunk = std::max(3.6, 3.9 * m + 0.07 * m * m);
     steps = 3 + 1.2 * m + t * (0.9 + 0.02 * m);
   }
-  return 1.05 * (launch + n * chunk) < steps;
+  return 1.03 * (launch + n * chunk) < steps;
 }
 
 DnChunkWs dn_chunk_ws(void* workspace, int64_t rows, int64_t nch, int64_t heads, int64_t qk_heads,

@@ -32,8 +32,8 @@ def test_calls_that_stay_step_by_step(need, rows, t, out, heads) -> None:
 
 
 @pytest.mark.parametrize("rows,t,out,heads", [
-    # 35 / 29, 57 / 44, 107 / 69, 207 / 116, 400 / 314, 2286 / 178
-    (1, 24, True, 64), (2, 40, True, 64), (4, 64, True, 64), (4, 128, True, 64), (8, 256, True, 64), (1, 1500, True, 64),
+    # 35 / 29, 57 / 44, 68 / 56, 82 / 68, 106 / 95, 107 / 69, 207 / 116, 400 / 314, 2286 / 178
+    (1, 24, True, 64), (2, 40, True, 64), (3, 40, True, 64), (4, 48, True, 64), (6, 64, True, 64), (4, 64, True, 64), (4, 128, True, 64), (8, 256, True, 64), (1, 1500, True, 64),
     # 34 / 25, 42 / 33, 76 / 51, 149 / 131, 1637 / 116
     (1, 32, False, 64), (2, 40, False, 64), (4, 64, False, 64), (8, 128, False, 64), (1, 1500, False, 64),
     (1, 24, True, 4), (1, 32, False, 4),
